@@ -48,20 +48,41 @@ struct prism_hip_model {
   hipStream_t cap_stream = nullptr;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
+  // Steps that may still run: on the context's stream, on streams of the caller's.
+  bool steps_own = false, steps_lent = false;
   std::vector<void*> allocs;
 };
 
-static void model_detach(prism_hip_model* m) { m->ctx = nullptr; }
+// (the context is being destroyed, which waits for its stream)
+static void model_detach(prism_hip_model* m) {
+  m->ctx = nullptr;
+  m->steps_own = false;
+}
 
 namespace {
 
 size_t payload4(uint32_t rows, uint32_t k) { return (size_t)rows * 32 + (size_t)rows * (k / 2); }
 
+// Waits for the model's steps: their executable, and the kernel arguments it
+// owns, are destroyed only after it.  The caller's streams may be gone by now,
+// so steps on those are waited for with the whole device.
+hipError_t model_wait(prism_hip_model* m) {
+  hipError_t e = hipSuccess;
+  if (m->steps_lent)
+    e = hipDeviceSynchronize();
+  else if (m->steps_own)
+    e = hipStreamSynchronize(m->ctx->stream);
+  if (e == hipSuccess) m->steps_own = m->steps_lent = false;
+  return e;
+}
+
 void model_release(prism_hip_model* m) {
   DeviceGuard g(m->device);
-  if (m->exec) (void)hipGraphExecDestroy(m->exec);
-  if (m->graph) (void)hipGraphDestroy(m->graph);
-  if (m->cap_stream) (void)hipStreamDestroy(m->cap_stream);
+  if (model_wait(m) == hipSuccess) {  // (else they are left, not destroyed under a running step)
+    if (m->exec) (void)hipGraphExecDestroy(m->exec);
+    if (m->graph) (void)hipGraphDestroy(m->graph);
+    if (m->cap_stream) (void)hipStreamDestroy(m->cap_stream);
+  }
   for (void* p : m->allocs) (void)hipFree(p);
   m->allocs.clear();
   m->exec = nullptr;
@@ -78,6 +99,7 @@ int model_alloc(prism_hip_model* m, T** p, size_t bytes) {
   return PRISM_HIP_OK;
 }
 
+// (no step runs: the caller has called model_wait)
 void model_invalidate(prism_hip_model* m) {
   if (m->exec) (void)hipGraphExecDestroy(m->exec);
   if (m->graph) (void)hipGraphDestroy(m->graph);
@@ -250,6 +272,7 @@ int prism_hip_model_set_embedding(prism_hip_model* m, const prism_hip_weight* em
   prism_hip_ctx* ctx = m->ctx;
   if ((rc = check_w4(ctx, embed, "embedding", m->cfg.vocab, m->cfg.hidden))) return rc;
   DeviceGuard g(m->device);
+  HIP_TRY(ctx, model_wait(m));
   if ((rc = copy_split_rows(ctx, embed, m->embed, m->embed + (size_t)m->cfg.vocab * 32, ctx->stream))) return rc;
   HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
   m->embed_set = true;
@@ -274,6 +297,7 @@ int prism_hip_model_set_layer(prism_hip_model* m, uint32_t layer, const prism_hi
       (rc = check_w4(ctx, down_proj, "down_proj", D, I)))
     return rc;
   DeviceGuard g(m->device);
+  HIP_TRY(ctx, model_wait(m));
   hipStream_t st = ctx->stream;
   // fused QKV: LUT rows q|k|v, then index rows q|k|v
   uint8_t* f = m->qkv[layer];
@@ -416,6 +440,7 @@ int prism_hip_model_step_dev(prism_hip_model* m, uint32_t token, int64_t pos, vo
   hipLaunchKernelGGL(prism::k_step_begin, dim3(1), dim3(256), 0, st, p, m->d_params, m->embed, c.vocab, c.hidden,
                      m->hres);
   HIP_TRY(ctx, hipGetLastError());
+  (st == ctx->stream ? m->steps_own : m->steps_lent) = true;
   HIP_TRY(ctx, hipGraphLaunch(m->exec, st));
   for (uint32_t l = 0; l < c.n_layers; l++) m->kv_len[l] += 1;
   ctx->err.clear();

@@ -1,11 +1,14 @@
-"""What Model.logits_dev() returns keeps the model's memory alive: a tensor over
-the logits was left with freed device memory once the last reference to the
-Model was gone."""
+"""The life of a model's device memory.  What Model.logits_dev() returns keeps it
+alive: a tensor over the logits was left with freed device memory once the last
+reference to the Model was gone, or close() was called.  And a step that still
+runs keeps its graph: it was destroyed before anything waited for the step."""
 import gc
 import types
 
 import numpy as np
 import pytest
+
+import fake_hip
 
 
 def test_logits_address_keeps_the_model(pe):
@@ -40,3 +43,48 @@ def test_logits_tensor_outlives_the_model_reference(pe, gpu_ctx):
     del m
     gc.collect()
     assert np.array_equal(logits.cpu().numpy().view(np.uint16), want.view(np.uint16))
+
+
+# ---- the order of waits and destructions, with the fake runtime
+
+STREAM = 0x77000  # a stream of the caller's
+
+
+def _model(hip, pe):
+    cfg = pe.Qwen2Config(n_layers=1, hidden=128, n_heads=2, n_kv_heads=1, intermediate=64, vocab=304)
+    ctx = pe.Context(0)
+    m = pe.Model(ctx, cfg, max_seq=8)
+
+    def upload(n, k):
+        nbytes = n * 32 + n * k // 2
+        return ctx.upload_dev(fake_hip.Tensor(hip, nbytes), n, k, 4)
+
+    m.set_embedding(upload(cfg.vocab, cfg.hidden))
+    layer = [upload(n, k) for n, k in cfg.shapes().values()]
+    m.set_layer(0, layer)
+    hip.clear()
+    return ctx, m, layer
+
+
+def release_in_flight(hip, pe, stream, how):
+    ctx, m, layer = _model(hip, pe)
+    m.step_dev(3, 0, stream)
+    if how == "close":
+        m.close()
+    elif how == "new weights":
+        m.set_layer(0, layer)
+    elif how == "context first":
+        ctx.close()
+        m.close()
+    return hip.log()
+
+
+@pytest.mark.parametrize("stream", [None, STREAM])
+@pytest.mark.parametrize("how", ["close", "new weights", "context first"])
+def test_a_step_in_flight_is_waited_for(stream, how):
+    """A model that is freed or gets new weights while a step runs, on the
+    context's stream or the caller's: its executable, graph and capture stream
+    are destroyed after a wait that covers the step."""
+    log = fake_hip.call(__name__, "release_in_flight", stream, how)
+    assert any(ln.startswith("graph launch") for ln in log) and any(ln.startswith("exec destroy") for ln in log)
+    assert not [ln for ln in log if ln.endswith("IN FLIGHT")], log
