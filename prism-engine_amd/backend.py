@@ -249,12 +249,27 @@ class Weight:
             pass
 
 
-class _ModelAddress(int):
-    """An address in a model's device memory, with a reference to the model."""
+class _ModelHandle:
+    """Owns a prism_hip_model: it is freed when the last reference goes."""
 
-    def __new__(cls, value: int, model: "Model"):
+    def __init__(self, lib, h):
+        self.lib, self.h = lib, h
+
+    def __del__(self):
+        if sys.is_finalizing():
+            return
+        try:
+            self.lib.prism_hip_model_free(self.h)
+        except Exception:
+            pass
+
+
+class _ModelAddress(int):
+    """An address in a model's device memory, with a reference to the model's handle."""
+
+    def __new__(cls, value: int, handle: _ModelHandle):
         self = super().__new__(cls, value)
-        self._model = model
+        self._handle = handle
         return self
 
 
@@ -268,6 +283,16 @@ class Model:
         self.h = ctx.lib.prism_hip_model_create(ctx.h, ctypes.byref(c))
         if not self.h:
             raise PrismHipError(_native.ERR_SHAPE, ctx.error())
+
+    _handle = None  # a _ModelHandle, while the model is open
+
+    @property
+    def h(self):
+        return self._handle.h if self._handle else None
+
+    @h.setter
+    def h(self, h) -> None:
+        self._handle = _ModelHandle(self.ctx.lib, h) if h else None
 
     @classmethod
     def from_tensors(cls, ctx: Context, cfg, embed: PalettizedTensor, layers, max_seq: int = 4096) -> "Model":
@@ -329,23 +354,15 @@ class Model:
         self.ctx.check(self.ctx.lib.prism_hip_model_step_dev(self.h, token, pos, _stream_handle(stream)))
 
     def logits_dev(self) -> int:
-        """Device address of the logits.  It keeps the model (and so the
-        memory) alive, and what holds it does: a tensor that wraps it may
-        outlive the caller's own reference to the model."""
-        return _ModelAddress(self.ctx.lib.prism_hip_model_logits_dev(self.h) or 0, self)
+        """Device address of the logits.  It keeps the model's memory alive,
+        and what holds it does: a tensor that wraps it may outlive the
+        caller's own reference to the model, and close()."""
+        return _ModelAddress(self.ctx.lib.prism_hip_model_logits_dev(self.h) or 0, self._handle)
 
     def close(self) -> None:
-        if self.h:
-            self.ctx.lib.prism_hip_model_free(self.h)
-            self.h = None
-
-    def __del__(self):
-        if sys.is_finalizing():
-            return
-        try:
-            self.close()
-        except Exception:
-            pass
+        """No calls from here on; the memory is freed with the last address of
+        logits_dev() that is still held."""
+        self.h = None
 
 
 class HipBackend:

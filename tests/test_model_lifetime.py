@@ -88,3 +88,29 @@ def test_a_step_in_flight_is_waited_for(stream, how):
     log = fake_hip.call(__name__, "release_in_flight", stream, how)
     assert any(ln.startswith("graph launch") for ln in log) and any(ln.startswith("exec destroy") for ln in log)
     assert not [ln for ln in log if ln.endswith("IN FLIGHT")], log
+
+
+def close_with_address(hip, pe):
+    ctx, m, _ = _model(hip, pe)
+    p = m.logits_dev()
+    held = {"data": (p, False)}
+    address = int(p)
+    m.close()
+    m.close()
+    with pytest.raises(pe.PrismHipError):
+        m.step_dev(3, 0)
+    open_, lines = hip.room(address), hip.log()
+    del p, m
+    gc.collect()
+    still = hip.room(address)
+    del held
+    gc.collect()
+    return [open_, still, hip.room(address), [ln for ln in lines if ln.startswith("free")]]
+
+
+def test_close_leaves_a_held_address_valid():
+    """close() while an address of logits_dev() is held: the memory stays until
+    the address is gone, and then it goes."""
+    closed, dropped, gone, frees = fake_hip.call(__name__, "close_with_address")
+    assert closed >= 608 and dropped >= 608 and frees == []
+    assert gone == 0
