@@ -1234,10 +1234,12 @@ int run_gemm(prism_hip_ctx* ctx, const prism_hip_weight* w, GemmPlan p, const vo
                             : prism::lkx_kernel(bits, p.tt, K % unit != 0);
   const uint32_t rows = p.packed ? 32u * p.rt : 64u;
   const uint32_t group = 32u * p.tt * (p.packed ? prism::kLkWaves / p.ks : 1u);
-  // index and LUT offsets are 31-bit: split-block weights past 2 GiB of either go in row slabs
+  // index and LUT offsets are 31-bit: split-block weights past 2 GiB of either go in row slabs.
+  // GI weights are below 2 GiB whole (gi_rows), and their rows lie in groups: never cut.
   const size_t row_bytes = (size_t)K * bits / 8;
-  const uint32_t slab =
-      (uint32_t)std::min<size_t>(N, kMaxIndexBytes / std::max<size_t>(row_bytes, 2u << bits) / rows * rows);
+  const uint32_t slab = w->gi ? N
+                              : (uint32_t)std::min<size_t>(
+                                    N, kMaxIndexBytes / std::max<size_t>(row_bytes, 2u << bits) / rows * rows);
   hipError_t e = slab ? hipSuccess : hipErrorInvalidValue;
   for (uint32_t m = 0; m < M && e == hipSuccess; m += p.tokens) {
     const uint16_t* X = static_cast<const uint16_t*>(d_X) + (size_t)m * K;

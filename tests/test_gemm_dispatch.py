@@ -1,0 +1,55 @@
+"""The GEMM's dispatch on the CPU, with the fake HIP runtime: which kernels a
+call launches and with which pointers, at sizes no GPU test can hold."""
+import pytest
+
+import fake_hip
+
+
+def payload_bytes(n, k, bits):
+    return n * (2 << bits) + n * k * bits // 8
+
+
+def launches(hip, pe, bits, n, k, ms, x_bytes=None):
+    """gemm_dev of each M: (layout's group rows, [kernel, rows, first row's LUT and index offset in the weight,
+    first row of Y] of each lookup launch, every kernel)."""
+    ctx = pe.Context(0)
+    w = ctx.upload_dev(fake_hip.Tensor(hip, payload_bytes(n, k, bits)), n, k, bits)
+    out = []
+    for m in ms:
+        x, y = fake_hip.Tensor(hip, m * k * 2), fake_hip.Tensor(hip, m * n * 2)
+        hip.clear()
+        ctx.gemm_dev(w, x, m, y)
+        lk = [ln for ln in hip.launches if ln.lk]
+        first = [ln.lk for ln in lk]
+        base = min((a.lut for a in first), default=0)
+        out.append({"G": first[0].G if first else 0, "kernels": [ln.name for ln in hip.launches],
+                    "lk": [[ln.name, ln.lk.N, ln.lk.lut - base, ln.lk.idx - base, (ln.lk.Y - y.address) // 2 % n]
+                           for ln in lk],
+                    "room": [[hip.room(a.lut), hip.room(a.idx), hip.room(a.X), hip.room(a.Y)] for a in first]})
+    return out
+
+
+# GI weights just below the layout's 2 GiB end, past the bytes a split-block slab takes:
+# 4-bit in 32-row groups (2 132 803 584 bytes), 8-bit in 32-row groups (2 139 095 040)
+@pytest.mark.parametrize("bits,n,k", [(4, 32768, 130112), (8, 8192, 260608)])
+def test_gi_weights_are_never_cut(bits, n, k):
+    """The rows of GI weights lie in groups, so a slab's first row is no
+    row-multiple from the base: one launch takes them all."""
+    for got in fake_hip.call(__name__, "launches", bits, n, k, [17, 300]):
+        assert got["G"] == 32
+        assert [x[1:] for x in got["lk"]] == [[n, 0, 0, 0]], got
+
+
+@pytest.mark.parametrize("bits,n,k", [(4, 33000, 130112), (8, 70000, 32768), (8, 4_200_003, 8)])
+def test_split_block_slabs(bits, n, k):
+    """Split-block weights past 2 GiB of index or LUT bytes: slabs of whole
+    tiles that cover every row once, each launch's bytes below 2 GiB."""
+    row, lut = k * bits // 8, 2 << bits
+    for got in fake_hip.call(__name__, "launches", bits, n, k, [17, 40]):
+        assert got["G"] == 0 and len(got["lk"]) > 1
+        at = 0
+        for _, rows, lut_at, idx_at, y_at in got["lk"]:
+            assert lut_at == at * lut and idx_at == n * lut + at * row and y_at == at
+            assert rows * max(row, lut) < 1 << 31 and (rows % 64 == 0 or at + rows == n)
+            at += rows
+        assert at == n
