@@ -1240,7 +1240,7 @@ int run_gemm(prism_hip_ctx* ctx, const prism_hip_weight* w, GemmPlan p, const vo
   const uint32_t slab = w->gi ? N
                               : (uint32_t)std::min<size_t>(
                                     N, kMaxIndexBytes / std::max<size_t>(row_bytes, 2u << bits) / rows * rows);
-  hipError_t e = slab ? hipSuccess : hipErrorInvalidValue;
+  hipError_t e = hipSuccess;
   for (uint32_t m = 0; m < M && e == hipSuccess; m += p.tokens) {
     const uint16_t* X = static_cast<const uint16_t*>(d_X) + (size_t)m * K;
     a.M = std::min(p.tokens, M - m);
@@ -1374,7 +1374,7 @@ GemmPlan plan_gemm(uint32_t bits, uint32_t M, uint32_t N, uint32_t K, uint32_t n
 }
 
 // Whether M tokens go to the lookup GEMM rather than to GEMV passes (rows in
-// eights, aligned x).  `gemv`: the GEMV entry points, whose GI calls of more
+// eights below 2^24, aligned x).  `gemv`: the GEMV entry points, whose GI calls of more
 // than 16 vectors stay with their passes.  MI355X, lookup against passes:
 //  * above 16 tokens always: two passes or more read the weights again
 //    (14336 x 4096, 32 tokens, 4 bits 10.9 against 24.7 us, 8 bits 19.9
@@ -1392,6 +1392,8 @@ GemmPlan plan_gemm(uint32_t bits, uint32_t M, uint32_t N, uint32_t K, uint32_t n
 bool lookup_takes(const prism_hip_ctx* ctx, const prism_hip_weight* w, const void* d_x, uint32_t M, bool gemv) {
   const uint32_t N = w->dim_m, K = w->dim_n;
   if (K % 8 != 0 || reinterpret_cast<uintptr_t>(d_x) % 16 != 0) return false;
+  // 31-bit offsets: 64 tokens of x (and with that a tile's rows of indices) below 2 GiB
+  if ((uint64_t)K * 64 * 2 >= (1ull << 31)) return false;
   if (M > 16) return !(gemv && w->gi);
   const bool mfma = K % prism::kGmGroup == 0 && (w->gi || N >= 4096);
   if (M >= 9) return !mfma || (K >= 4096 && (N + 63) / 64 <= (uint32_t)ctx->num_cu);

@@ -54,3 +54,15 @@ def test_split_block_slabs(bits, n, k):
             assert rows * max(row, lut) < 1 << 31 and (rows % 64 == 0 or at + rows == n)
             at += rows
         assert at == n
+
+
+@pytest.mark.parametrize("bits,n,k,taken", [(4, 3, (1 << 24) - 8, True), (8, 3, (1 << 24) - 8, True),
+                                            (4, 3, 1 << 24, False), (8, 3, 1 << 24, False), (4, 70, 1 << 25, False),
+                                            (8, 1, 1 << 26, False), (4, 2, 1 << 28, False)])
+def test_rows_past_the_offsets_go_to_passes(bits, n, k, taken):
+    """64 tokens of x from 2 GiB on, and row tiles past 2 GiB of indices: the
+    GEMV passes, which address them by 64-bit pointers."""
+    for got in fake_hip.call(__name__, "launches", bits, n, k, [17, 40, 64, 70]):
+        assert bool(got["lk"]) == taken and got["kernels"], got
+        for x in got["lk"]:
+            assert x[1] == n
