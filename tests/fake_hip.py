@@ -41,11 +41,18 @@ class LkArgs(ctypes.Structure):
                [(n, ctypes.c_uint32) for n in ("M", "N", "K", "ldy", "G", "per_split", "KS")]
 
 
-class Launch:
-    """One kernel launch; `lk`: the arguments of a lookup GEMM kernel."""
+# Arguments of other kernels that tests look at.
+PLAIN = {"k_pack_x": [("X", ctypes.c_uint64), ("Xp", ctypes.c_uint64), ("M", ctypes.c_uint32), ("K", ctypes.c_uint32),
+                      ("steps", ctypes.c_uint32), ("tiles", ctypes.c_uint32)],
+         "k_gemm_split_sum": [("P", ctypes.c_uint64), ("Y", ctypes.c_uint64), ("mn", ctypes.c_uint64),
+                              ("S", ctypes.c_uint32)]}
 
-    def __init__(self, name, grid, threads, stream, lk):
-        self.name, self.grid, self.threads, self.stream, self.lk = name, grid, threads, stream, lk
+
+class Launch:
+    """One kernel launch; `lk`: the arguments of a lookup GEMM kernel, `args`: of a kernel of PLAIN."""
+
+    def __init__(self, name, grid, threads, stream, lk, args):
+        self.name, self.grid, self.threads, self.stream, self.lk, self.args = name, grid, threads, stream, lk, args
 
 
 class Hip:
@@ -56,7 +63,7 @@ class Hip:
         lib.fake_set_capturing.argtypes = [ctypes.c_void_p]
         lib.fake_refuse.argtypes = [ctypes.c_size_t]
         lib.fake_room.restype, lib.fake_room.argtypes = ctypes.c_size_t, [ctypes.c_uint64]
-        self.launches = []
+        self.launches, self.on_append = [], None
         kind = ctypes.CFUNCTYPE(None, ctypes.c_char_p, ctypes.POINTER(ctypes.c_uint), ctypes.POINTER(ctypes.c_void_p),
                                 ctypes.c_void_p)
 
@@ -65,7 +72,11 @@ class Hip:
             lk = None
             if "k_gemm_lookup" in name:
                 lk = LkArgs.from_buffer_copy(ctypes.string_at(args[0], ctypes.sizeof(LkArgs)))
-            self.launches.append(Launch(name, (dims[0], dims[1]), dims[3], stream or 0, lk))
+            plain = next((v for k, v in PLAIN.items() if k in name), [])
+            values = {n: t.from_address(args[i]).value for i, (n, t) in enumerate(plain)}
+            self.launches.append(Launch(name, (dims[0], dims[1]), dims[3], stream or 0, lk, values))
+            if self.on_append:  # (a call's own scratch is gone once the call returns)
+                self.on_append(self.launches[-1])
 
         self._on_launch = kind(on_launch)
         lib.fake_on_launch(self._on_launch)

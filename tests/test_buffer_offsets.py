@@ -25,6 +25,8 @@ import re
 import numpy as np
 import pytest
 
+import fake_hip
+
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "prism-engine_amd", "csrc")
 
 
@@ -538,3 +540,249 @@ def test_gemv_lpr4q_offsets(N, K, nb):
         b, o = p // (K // 8), p % (K // 8)
         assert ((b * xrow + 4 * o + 4) <= LPR8M_XDW)[p < xq].all(), "x store leaves its LDS region"
     assert ((tid[:, None] + 512 * np.arange(8)[None, :]) < xq).sum() == xq, "x pieces cover x once"
+
+
+# ---- k_gemm_lookup, k_gemm_lookup_x and k_pack_x (gemm_lookup.hip), for the launches that the library makes
+def gemm_launches(hip, pe, bits, N, K, calls):
+    """Every launch of gemm_dev for each (M, "own" | "lent" | "capture" | "noalloc"): name, grid, arguments, and the
+    bytes from each pointer to the end of its allocation."""
+    ctx = pe.Context(0)
+    w = ctx.upload_dev(fake_hip.Tensor(hip, N * (2 << bits) + N * K * bits // 8), N, K, bits)
+    out = []
+    for M, how in calls:
+        x, y = fake_hip.Tensor(hip, M * K * 2), fake_hip.Tensor(hip, M * N * 2)
+        hip.clear()
+        stream = None if how == "own" else 0x77000
+        hip.lib.fake_set_capturing(stream if how == "capture" else None)
+
+        def pointers(ln):
+            a = {n: getattr(ln.lk, n) for n, _ in fake_hip.LkArgs._fields_} if ln.lk else dict(ln.args)
+            a["room"] = {n: hip.room(v) for n, v in a.items() if n in ("lut", "idx", "X", "Y", "P", "Xp")}
+            a["name"], a["grid"] = ln.name, ln.grid
+            return a
+
+        got = []
+        hip.on_append = lambda ln: got.append(pointers(ln))
+        (ctx.gemm_dev_noalloc if how == "noalloc" else ctx.gemm_dev)(w, x, M, y, stream)
+        hip.on_append = None
+        out.append(got)
+    return out
+
+
+def _lk_common(a, bits):
+    """(bytes of the LUT and index ranges, index bytes from a row's chunk to its next): both ranges inside the
+    allocation.  Their loads have no scalar offset, so the range check covers them whole."""
+    N, K, G = a["N"], a["K"], a["G"]
+    ri = gi_bytes(G, N, K, bits) if G else N * (K * bits // 8)
+    rl = ri if G else N * (2 << bits)
+    assert ri < 1 << 31 and rl < 1 << 31, "31-bit ranges"
+    assert rl <= a["room"]["lut"] and ri <= a["room"]["idx"], "the descriptors end in the allocation"
+    return rl, ri, (G or 1) * GI_CHUNK
+
+
+def _lk_weights(a, bits, n0, rows, s0, s1, ahead, ri, rl, cstride):
+    """One wave's LUT and index loads: rows n0 .. n0 + rows, steps s0 .. s1 + ahead (from s1 on marked out of
+    range when `ahead`)."""
+    N, K, G = a["N"], a["K"], a["G"]
+    r = np.minimum(n0 + np.arange(rows), N - 1)
+    lut = np.array([gi_lut(G, int(v), K, bits) if G else int(v) * (2 << bits) for v in r])
+    assert (lut + (2 << bits) <= rl).all(), "LUT row"
+    chunk0 = np.array([gi_chunk_offset(G, int(v), 0, K, bits) if G else int(v) * (K * bits // 8) for v in r])
+    epc, chunks = 128 // bits, -(-K // (128 // bits))
+    for h in range(2):
+        s = np.array(sorted(set(range(s0, min(s1, s0 + 3))) | set(range(max(s0, s1 - 3), s1 + ahead))), dtype=np.int64)[None, :]
+        voff = (chunk0[:, None] + h * cstride + s * 2 * cstride) | np.where(s < s1, 0, 0x80000000)
+        performed = voff < ri
+        assert not performed[:, s[0] >= s1].any(), "steps past the wave's are not loaded"
+        # inside K every 16-byte chunk begins in the lane's own row; what lies past K is masked by the kernel
+        inside = (2 * s + h) < chunks
+        at = chunk0[:, None] + (2 * s + h) * cstride
+        assert ((voff == at) & performed | ~inside | (s >= s1)).all()
+        whole = (2 * s + h + 1) * epc <= K
+        assert ((voff + 16 <= ri) | ~whole | (s >= s1)).all(), "a whole chunk ends in the range"
+
+
+def gi_lut(G, r, K, bits):
+    return (r // G) * gi_group_bytes(G, K, bits) + (r % G) * (2 << bits)
+
+
+def _some(n):
+    """Some of n blocks: the first and last ones, and a few others."""
+    return sorted(set(range(min(n, 3))) | set(range(max(0, n - 3), n)) | set(np.random.default_rng(n).integers(0, n, 3).tolist()))
+
+
+def _lk_tile(t, tiles):
+    per, rem, xcd = tiles // 8, tiles % 8, t % 8
+    return xcd * per + min(xcd, rem) + t // 8
+
+
+def check_lookup_x(a, bits, TT, ragged):
+    N, K, M, per_split = a["N"], a["K"], a["M"], a["per_split"]
+    SK, R, MT = 256 // bits, 64, 32 * TT
+    PIECES, TPI = SK // 8, 64 // (SK // 8)
+    steps, nmb = -(-K // SK), -(-M // MT)
+    assert ragged == (K % SK != 0) and a["grid"][0] == nmb * -(-N // R) and a["grid"][1] == -(-steps // per_split)
+    assert sorted(_lk_tile(t, a["grid"][0]) for t in range(a["grid"][0])) == list(range(a["grid"][0]))
+    rl, ri, cstride = _lk_common(a, bits)
+    lane = np.arange(64)
+    for t in _some(a["grid"][0]):
+        n0, m0 = t // nmb * R, t % nmb * MT
+        live = min(M - m0, MT)
+        x_range = live * K * 2
+        assert x_range < 1 << 31 and m0 * K * 2 + x_range <= a["room"]["X"], "the x descriptor"
+        for by in _some(a["grid"][1]):
+            sb = by * per_split
+            ns = min(steps - sb, per_split)
+            cuts = [sb + w * ns // 8 for w in range(9)]
+            assert ns > 0 and cuts[0] == sb and cuts[8] == sb + ns
+            for w in (0, 7):
+                s0, s1 = cuts[w], cuts[w + 1]
+                _lk_weights(a, bits, n0, R, s0, s1, 0, ri, rl, cstride)
+                xk = 8 * (lane % PIECES)
+                for s in sorted({s0, s1 - 1} & set(range(s0, s1))):
+                    for i in range(MT // TPI):
+                        voff = np.where(s * SK + xk < K, (lane // PIECES) * K * 2 + xk * 2 + s * SK * 2 + i * TPI * K * 2,
+                                        0x80000000)
+                        performed = _check(voff, 0, 16, x_range, x_range, "lookup_x x")
+                        token = lane // PIECES + i * TPI
+                        assert (performed == ((token < live) & (s * SK + xk < K))).all()
+                        assert (voff + 16 <= (token + 1) * K * 2)[performed].all(), "x leaves its token"
+            # stores: partials [split][M][N], or Y [M][ldy]
+            _lk_stores(a, n0, R, m0, live, by)
+    # LDS dwords: the tables, then each wave's tokens; then the partial tiles
+    XP, RP = SK // 2 + 4, R + 4
+    size = max(256 * 64 + 8 * MT * XP, 8 * MT * RP)
+    assert size * 4 <= 160 << 10
+    assert ((lane // PIECES) * XP + 4 * (lane % PIECES)).max() + 4 + (MT // TPI - 1) * TPI * XP <= MT * XP
+    assert (lane % 32 * XP + lane // 32 * (128 // bits // 2)).max() + 32 * (TT - 1) * XP + 4 * (SK // 16 - 1) + 4 <= MT * XP
+
+
+def _lk_stores(a, n0, rows, m0, live, by):
+    last_r, last_m = min(n0 + rows, a["N"]) - 1, m0 + live - 1
+    if a["P"]:
+        assert (((by * a["M"] + last_m) * a["N"] + last_r) + 1) * 4 <= a["room"]["P"]
+    else:
+        assert (last_m * a["ldy"] + last_r + 1) * 2 <= a["room"]["Y"]
+
+
+def check_lookup(a, bits, RT, TT, ragged):
+    N, K, M, KS, per_split = a["N"], a["K"], a["M"], a["KS"], a["per_split"]
+    SK, R, TM, TG = 256 // bits, 32 * RT, 32 * TT, 8 // a["KS"]
+    NJ = SK // 16
+    pairs, nmb = -(-K // (2 * SK)), -(-M // (TM * TG))
+    steps = 2 * pairs
+    assert ragged == (K % (2 * SK) != 0) and KS in (1, 2, 4, 8)
+    assert a["grid"][0] == nmb * -(-N // R) and a["grid"][1] == -(-pairs // per_split)
+    rl, ri, cstride = _lk_common(a, bits)
+    tiles, tbytes = -(-M // 32), steps * NJ * 1024
+    ahead = (1 if bits == 4 and RT * TT > 4 else 2) + 1  # load_x(s + BD), load_i(s + 2)
+    lane = np.arange(64)
+    for t in _some(a["grid"][0]):
+        n0 = t // nmb * R
+        for by in _some(a["grid"][1]):
+            pb = by * per_split
+            n_pairs = min(pairs - pb, per_split)
+            assert n_pairs > 0
+            taken = []
+            for w in range(8):
+                ks, tg = w % KS, w // KS
+                m0 = t % nmb * TM * TG + tg * TM
+                s0 = 2 * (pb + ks * n_pairs // KS)
+                s1 = 2 * (pb + (ks + 1) * n_pairs // KS) if m0 < M else s0
+                u0 = m0 // 32
+                lt = min(tiles - u0, TT) if u0 < tiles else 0
+                assert (lt > 0) == (m0 < M)
+                if tg == 0:
+                    taken += range(s0, s1)
+                if w in (0, 7):
+                    _lk_weights(a, bits, n0, R, s0, s1, ahead, ri, rl, cstride)
+                base = (u0 if lt else 0) * tbytes
+                for s in {s0, max(s0, s1 - 1), s1, s1 + ahead - 1}:
+                    for u in range(TT):
+                        voff = (u * tbytes + lane * 16) | (0 if s < s1 else 0x80000000)
+                        for j in (0, NJ - 1):
+                            performed = _check(voff, (s * NJ + j) * 1024, 16, lt * tbytes, a["room"]["X"] - base, "lookup x")
+                            assert (performed == (s < s1 and u < lt)).all()
+                            if s < s1:  # the operands of (tile, step, j) as k_pack_x lays them out
+                                assert s < steps and ((u * tbytes + (s * NJ + j) * 1024 + 1024) <= (u + 1) * tbytes)
+                if m0 < M:
+                    _lk_stores(a, n0, R, m0, min(M - m0, TM), by)
+            assert taken == list(range(2 * pb, 2 * (pb + n_pairs))), "the K slices cover the split once"
+
+
+def check_pack(a, bits):
+    M, K, steps, tiles = a["M"], a["K"], a["steps"], a["tiles"]
+    SK = 256 // bits
+    PC, NJ = SK // 8, SK // 16
+    pieces = tiles * 32 * steps * PC
+    assert tiles == -(-M // 32) and a["grid"][0] == -(-pieces // 256) and pieces < 1 << 32 and K % 8 == 0
+    i = np.unique(np.concatenate([np.arange(min(pieces, 4096)), np.arange(max(0, pieces - 4096), pieces + 255),
+                                  np.random.default_rng(K).integers(0, pieces, 4096)]))
+    o, n, ts = i % PC, i // PC % 32, i // (32 * PC)
+    s, u = ts % steps, ts // steps
+    keep = u < tiles
+    m, k = u * 32 + n, s * SK + 8 * o
+    read = keep & (m < M) & (k < K)
+    assert ((m * K + k + 8) * 2 <= a["room"]["X"])[read].all()
+    h, j = o // (PC // 2), o % (PC // 2)
+    at = ((ts * NJ + j) * 64 + 32 * h + n) * 16
+    assert (at + 16 <= a["room"]["Xp"])[keep].all()
+    # k_gemm_lookup's operand (step s, MFMA j, lane 32 h + n) holds k = s SK + h EPC + 8 j ..
+    assert (k == s * SK + h * (SK // 2) + 8 * j).all()
+    assert len(np.unique(at[keep])) == keep.sum(), "every piece has a place of its own"
+
+
+def check_gemm_launches(launches, bits, M, N):
+    seen = set()
+    for a in launches:
+        m = re.search(r"(k_gemm_lookup_x|k_gemm_lookup|k_pack_x|k_gemm_split_sum)(?:<([^>]*)>)?", a["name"])
+        if not m:
+            continue
+        seen.add(m.group(1))
+        targs = [v.strip() for v in (m.group(2) or "").split(",")]
+        if m.group(1) == "k_gemm_lookup_x":
+            check_lookup_x(a, bits, int(targs[1]), targs[2] == "true")
+        elif m.group(1) == "k_gemm_lookup":
+            check_lookup(a, bits, int(targs[1]), int(targs[2]), targs[3] == "true")
+        elif m.group(1) == "k_pack_x":
+            check_pack(a, bits)
+        else:
+            assert a["mn"] == M * N and a["S"] * a["mn"] * 4 <= a["room"]["P"] and a["mn"] * 2 <= a["room"]["Y"]
+            assert a["grid"][0] * 1024 >= a["mn"]
+    return seen
+
+
+LK_CALLS = [(M, how) for M in (9, 33, 64, 65, 203, 512, 1030) for how in ("own", "lent", "capture", "noalloc")]
+
+
+# GI (both widths; 24-row tail groups), split-block, ragged K at both widths, few rows, long rows, an LM head
+@pytest.mark.parametrize("bits,N,K", [(4, 14336, 4096), (4, 9100, 2112), (4, 4096, 14336), (4, 1001, 1032), (4, 3, 8),
+                                      (4, 151936, 896), (4, 64, 16384), (4, 18944, 3584), (4, 257, 72), (8, 14336, 4096),
+                                      (8, 9100, 2048), (8, 4096, 14336), (8, 1001, 1032), (8, 5, 8), (8, 255, 40),
+                                      (8, 151936, 896), (8, 64, 16384)])
+def test_lookup_gemm_offsets(bits, N, K):
+    seen = set()
+    for (M, how), got in zip(LK_CALLS, fake_hip.call(__name__, "gemm_launches", bits, N, K, LK_CALLS)):
+        seen |= check_gemm_launches(got, bits, M, N)
+    assert "k_gemm_lookup_x" in seen
+
+
+def test_lookup_gemm_offsets_of_many_shapes():
+    """Shapes all over the range that a projection has, odd ones among them."""
+    rng = np.random.default_rng(7)
+    for bits in (4, 8):
+        for _ in range(10):
+            N, K = (int(2 ** v) for v in (rng.uniform(3, 14.5), rng.uniform(3, 14)))
+            K = K // 8 * 8 if rng.random() < 0.5 else max(128, K // 128 * 128)
+            calls = [(int(2 ** rng.uniform(3.2, 11)), how) for how in ("own", "lent", "capture", "noalloc") for _ in range(3)]
+            for (M, _), got in zip(calls, fake_hip.call(__name__, "gemm_launches", bits, N, K, calls)):
+                check_gemm_launches(got, bits, M, N)
+
+
+@pytest.mark.parametrize("bits,N,K", [(4, 32768, 130112), (8, 8192, 260608), (4, 33000, 130112), (8, 4_200_003, 8),
+                                      (4, 3, (1 << 24) - 8), (8, 70, (1 << 24) - 8)])
+def test_lookup_gemm_offsets_at_the_31_bit_ends(bits, N, K):
+    """GI weights just below 2 GiB, split-block slabs, the longest rows."""
+    calls = [(M, how) for M in (17, 64, 300) for how in ("own", "lent", "noalloc")]
+    for (M, _), got in zip(calls, fake_hip.call(__name__, "gemm_launches", bits, N, K, calls)):
+        assert check_gemm_launches(got, bits, M, N)
