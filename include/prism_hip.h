@@ -158,8 +158,10 @@ int prism_hip_gemm_dev(prism_hip_ctx* ctx, const prism_hip_weight* w, const void
 /* prism_hip_gemm_dev without any allocation.  No counterpart in the
  * reference: it is for callers that cannot allocate device memory (code
  * under HIP graph capture, serving loops, harnesses that forbid hipMalloc).
- * Same kernels and results as prism_hip_gemm_dev; its scratch is a static 64
- * MiB array on each GPU instead, which no call exceeds.  All calls on one GPU
+ * Same kernels and results as prism_hip_gemm_dev on the context's stream, on
+ * any stream (there prism_hip_gemm_dev pays for its scratch on each call and
+ * may split K otherwise); its scratch is a static 64 MiB array on each GPU
+ * instead, which no call exceeds.  All calls on one GPU
  * share that array: calls that overlap on one GPU (other streams, other
  * contexts) race. */
 int prism_hip_gemm_dev_noalloc(prism_hip_ctx* ctx, const prism_hip_weight* w, const void* d_X, uint32_t M,

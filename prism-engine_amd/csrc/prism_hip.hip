@@ -1404,8 +1404,8 @@ bool lookup_takes(const prism_hip_ctx* ctx, const prism_hip_weight* w, const voi
 int launch_gemm(prism_hip_ctx* ctx, const prism_hip_weight* w, const void* d_X, uint32_t M, void* d_Y,
                 hipStream_t st, float* fixed = nullptr) {
   if (!lookup_takes(ctx, w, d_X, M, false)) return launch_gemv_passes(ctx, w, nullptr, d_X, M, d_Y, st);
-  return run_gemm(ctx, w, plan_gemm(w->bits, M, w->dim_m, w->dim_n, (uint32_t)ctx->num_cu, st != ctx->stream), d_X, M,
-                  d_Y, st, fixed);
+  const bool lent = !fixed && st != ctx->stream;
+  return run_gemm(ctx, w, plan_gemm(w->bits, M, w->dim_m, w->dim_n, (uint32_t)ctx->num_cu, lent), d_X, M, d_Y, st, fixed);
 }
 
 // prism_hip_gemv and its like: several vectors may be the lookup GEMM's.

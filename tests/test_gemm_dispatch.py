@@ -66,3 +66,41 @@ def test_rows_past_the_offsets_go_to_passes(bits, n, k, taken):
         assert bool(got["lk"]) == taken and got["kernels"], got
         for x in got["lk"]:
             assert x[1] == n
+
+
+STREAM = 0x77000  # a stream of the caller's
+
+
+def plans(hip, pe, bits, n, k, ms, hows):
+    """For each M and each of "own", "lent", "capture", "noalloc own", "noalloc lent" (gemm_dev, gemm_dev_noalloc) and
+    "gemv own", "gemv lent", "gemv capture": [kernel, grid, K per split] of each launch, and the allocations and frees."""
+    ctx = pe.Context(0)
+    w = ctx.upload_dev(fake_hip.Tensor(hip, payload_bytes(n, k, bits)), n, k, bits)
+    out = []
+    for m in ms:
+        x, y = fake_hip.Tensor(hip, m * k * 2), fake_hip.Tensor(hip, m * n * 2)
+        row = {}
+        for how in hows:
+            hip.clear()
+            stream = None if how.endswith("own") else STREAM
+            hip.lib.fake_set_capturing(STREAM if how.endswith("capture") else None)
+            if how.startswith("noalloc"):
+                ctx.gemm_dev_noalloc(w, x, m, y, stream)
+            elif how.startswith("gemv"):
+                ctx.gemv_dev(w, x, m, y, stream)
+            else:
+                ctx.gemm_dev(w, x, m, y, stream)
+            row[how] = {"kernels": [[ln.name.replace("prism::", "").replace("void ", "").split("(")[0], ln.grid,
+                                     ln.lk.per_split if ln.lk else 0] for ln in hip.launches],
+                        "memory": [ln for ln in hip.log() if "malloc" in ln or "free" in ln]}
+        out.append(row)
+    return out
+
+
+@pytest.mark.parametrize("bits,n,k", [(4, 4096, 14336), (4, 14336, 4096), (8, 4096, 14336), (4, 2000, 2048)])
+def test_noalloc_is_planned_without_a_price_for_scratch(bits, n, k):
+    """The static scratch costs nothing, so a caller's stream gets the plan of
+    the context's."""
+    for row in fake_hip.call(__name__, "plans", bits, n, k, [24, 64, 96, 200, 300], ["own", "noalloc own", "noalloc lent"]):
+        assert row["noalloc lent"]["kernels"] == row["noalloc own"]["kernels"] == row["own"]["kernels"]
+        assert row["noalloc lent"]["memory"] == []

@@ -1,9 +1,9 @@
-"""prism_hip_gemm_dev_noalloc (the GEMM entry point that allocates nothing)
-against prism_hip_gemm_dev, through the C ABI.
+"""prism_hip_gemm_dev_noalloc (the GEMM entry point that allocates nothing) on
+a caller's stream against prism_hip_gemm_dev on the context's, through the C ABI.
 
-Both run the same kernels with the same split-K plan; only where the fp32
+Both run the same kernels with the same plan; only where packed X and the fp32
 partials live differs (the library's static per-GPU scratch instead of the
-context's pool), so the outputs must be bit-identical.  Each case makes two
+context's buffer), so the outputs must be bit-identical.  Each case makes two
 calls in a row, the second with fewer rows of X, so a stale first call's
 partials in the shared scratch would show in the second.
 """
@@ -12,21 +12,23 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
-# (bits, N, K, M first call, M second call): split-K 4-bit (4 and 2 splits),
-# GI and split-block device layouts, split-K 8-bit, an unsplit prefill and
-# the GEMV path (no partials at all).
+# (bits, N, K, M first call, M second call, the kernel of the first call that uses
+# scratch): X packed (GI and split-block layouts), K split with X as it is and
+# packed, and calls without scratch.
 CASES = [
-    (4, 14336, 4096, 256, 64),
-    (4, 2000, 2048, 200, 96),
-    (4, 4864, 896, 128, 40),
-    (8, 14336, 4096, 200, 65),
-    (4, 4096, 1024, 600, 520),
-    (4, 1024, 512, 24, 9),
+    (4, 14336, 4096, 256, 64, "k_pack_x"),
+    (4, 2000, 2048, 200, 96, None),
+    (4, 4864, 896, 128, 40, None),
+    (8, 14336, 4096, 200, 65, "k_pack_x"),
+    (4, 4096, 1024, 600, 520, None),
+    (4, 1024, 512, 24, 9, None),
+    (4, 4096, 14336, 40, 24, "k_gemm_split_sum"),
+    (4, 1024, 16384, 300, 200, "k_gemm_split_sum"),
 ]
 
 
-@pytest.mark.parametrize("bits,N,K,M1,M2", CASES)
-def test_gemm_noalloc_matches_gemm_dev(pe, gpu_ctx, bits, N, K, M1, M2):
+@pytest.mark.parametrize("bits,N,K,M1,M2,scratch", CASES)
+def test_gemm_noalloc_matches_gemm_dev(pe, gpu_ctx, bits, N, K, M1, M2, scratch):
     import torch
     print(f"[no_alloc] bits={bits} N={N} K={K} M={M1},{M2}", flush=True)
     t = pe.synth_tensor(N, K, bits, seed=N + K + bits)
@@ -38,9 +40,12 @@ def test_gemm_noalloc_matches_gemm_dev(pe, gpu_ctx, bits, N, K, M1, M2):
         want = torch.full((M, N), -1, dtype=torch.int16, device="cuda")
         got = torch.full((M, N), -2, dtype=torch.int16, device="cuda")
         torch.cuda.synchronize()
-        gpu_ctx.gemm_dev(w, dX, M, want, s)
+        gpu_ctx.gemm_dev(w, dX, M, want)
         gpu_ctx.gemm_dev_noalloc(w, dX, M, got, s)
         s.synchronize()
+        gpu_ctx.synchronize()
+        if i == 0 and scratch:
+            assert scratch in gpu_ctx.last_kernels()
         a = want.cpu().numpy()
         b = got.cpu().numpy()
         assert np.array_equal(a, b), (f"call {i}: M={M}: {int(np.sum(a != b))} of {a.size} outputs differ "
@@ -93,8 +98,8 @@ def test_gemm_noalloc_replayed_from_a_hip_graph(pe, gpu_ctx):
         with torch.cuda.stream(s):
             g.replay()
         s.synchronize()
-        gpu_ctx.gemm_dev(w, dX, M, want, s)
-        s.synchronize()
+        gpu_ctx.gemm_dev(w, dX, M, want)
+        gpu_ctx.synchronize()
         a, b = want.cpu().numpy(), dY.cpu().numpy()
         assert np.array_equal(a, b), f"replay {i}: {int(np.sum(a != b))} of {a.size} outputs differ"
     del g
