@@ -150,8 +150,10 @@ int prism_hip_gate_up_dev(prism_hip_ctx* ctx, const prism_hip_weight* gate, cons
  * range; up to 64 MiB): calls on the context's stream share a buffer that the
  * context keeps, a call on another stream takes its own from a stream-ordered
  * pool that the context creates on first use and frees it on that stream, so
- * calls on different streams do not share any.  Without memory for it the
- * call runs on a kernel that needs none. */
+ * calls on different streams do not share any.  Without memory for it, and
+ * while the stream is being captured, the call runs on a kernel that needs
+ * none (a captured call is kernels alone; prism_hip_gemm_dev_noalloc captures
+ * the others too, which long 8-bit prefills run twice as fast on). */
 int prism_hip_gemm(prism_hip_ctx* ctx, const prism_hip_weight* w, const uint16_t* X, uint32_t M, uint16_t* Y);
 int prism_hip_gemm_dev(prism_hip_ctx* ctx, const prism_hip_weight* w, const void* d_X, uint32_t M, void* d_Y,
                        void* stream);
@@ -161,9 +163,8 @@ int prism_hip_gemm_dev(prism_hip_ctx* ctx, const prism_hip_weight* w, const void
  * Same kernels and results as prism_hip_gemm_dev on the context's stream, on
  * any stream (there prism_hip_gemm_dev pays for its scratch on each call and
  * may split K otherwise); its scratch is a static 64 MiB array on each GPU
- * instead, which no call exceeds.  All calls on one GPU
- * share that array: calls that overlap on one GPU (other streams, other
- * contexts) race. */
+ * instead, which no call exceeds.  All calls on one GPU share that array:
+ * calls that overlap on one GPU (other streams, other contexts) race. */
 int prism_hip_gemm_dev_noalloc(prism_hip_ctx* ctx, const prism_hip_weight* w, const void* d_X, uint32_t M,
                                void* d_Y, void* stream);
 

@@ -1200,7 +1200,7 @@ int run_gemm(prism_hip_ctx* ctx, const prism_hip_weight* w, GemmPlan p, const vo
   const uint32_t N = w->dim_m, K = w->dim_n, bits = w->bits, step = prism::lk_step(bits);
   const size_t need = p.x_bytes + p.p_bytes;
   // scratch: the caller's, the context stream's kept one, or on another
-  // stream (or under its capture) one of the call's own from the pool
+  // stream one of the call's own from the pool
   void* scratch_mem = fixed;
   bool temp = false;
   if (need && !fixed) {
@@ -1308,20 +1308,23 @@ float gemm_w4_us(int mi, uint32_t M, uint32_t N, uint32_t K, uint32_t num_cu) {
   return (float)((tiles + num_cu - 1) / num_cu) * ((mi == 8 ? 6.5f : 8.5f) + step * (float)(K / prism::GW4_BK));
 }
 
+// Where a call's scratch (packed X, partials) comes from: kept memory, the pool
+// for this call, or none may be used.
+enum class Scratch { kKept, kCall, kNone };
+
 // The fastest plan by that estimate.  k_gemm_lookup_x up to 256 tokens (X
 // unpacked costs no launch: 14336 x 4096, 33 tokens 15 us; but 128 tokens 32
-// against 23.4), k_gemm_lookup above 64.  `lent`: a stream of the caller's,
-// where scratch is allocated and freed on each call, about 22 us of host
-// time.  4-bit calls of 49..64 tokens whose row blocks fit the CUs always
+// against 23.4), k_gemm_lookup above 64.  Scratch of the
+// call's own is allocated and freed on each call, about 22 us of host time.  4-bit calls of 49..64 tokens whose row blocks fit the CUs always
 // split K: tests/test_zz_no_alloc.py holds 64 tokens of 14336 x 4096 to a plan
 // with partials, though it is the slower one there (22.9 against 15.6 us
 // unsplit).
-GemmPlan plan_gemm(uint32_t bits, uint32_t M, uint32_t N, uint32_t K, uint32_t num_cu, bool lent) {
+GemmPlan plan_gemm(uint32_t bits, uint32_t M, uint32_t N, uint32_t K, uint32_t num_cu, Scratch scratch) {
   GemmPlan best;
   float best_us = 3.4e38f;
   // (weights that run_gemm cuts into row slabs have no partials)
   const uint32_t max_split = (uint64_t)N * K * bits / 8 < kMaxIndexBytes ? 16 : 1;
-  const uint32_t min_split = bits == 4 && M > 48 && M <= 64 && N <= 64 * num_cu ? 2 : 1;
+  const uint32_t min_split = scratch != Scratch::kNone && bits == 4 && M > 48 && M <= 64 && N <= 64 * num_cu ? 2 : 1;
   auto consider = [&](bool packed, int rt, int tt, uint32_t ks) {
     for (uint32_t split = min_split; split <= max_split; split *= 2) {
       GemmPlan p;
@@ -1331,15 +1334,16 @@ GemmPlan plan_gemm(uint32_t bits, uint32_t M, uint32_t N, uint32_t K, uint32_t n
       p.ks = ks;
       p.split = split;
       if (!plan_sizes(&p, bits, M, N, K)) continue;
+      if (scratch == Scratch::kNone && p.x_bytes + p.p_bytes) continue;
       float us = gemm_plan_us(p, bits, M, N, K, num_cu);
-      if (lent && p.x_bytes + p.p_bytes) us = std::max(us, 22.0f);
+      if (scratch == Scratch::kCall && p.x_bytes + p.p_bytes) us = std::max(us, 22.0f);
       if (us < best_us) {
         best_us = us;
         best = p;
       }
     }
   };
-  if (M <= 256) {
+  if (M <= 256 || scratch == Scratch::kNone) {
     consider(false, 2, 1, prism::kLkWaves);
     if (M > 32) consider(false, 2, 2, prism::kLkWaves);
   }
@@ -1401,30 +1405,36 @@ bool lookup_takes(const prism_hip_ctx* ctx, const prism_hip_weight* w, const voi
   return false;
 }
 
+// A call on the context's stream uses its buffer, one on a caller's stream memory
+// of its own, and under the capture of a caller's stream none: a captured call
+// is kernels alone, with no memory of its own in the graph.
+int scratch_of(prism_hip_ctx* ctx, hipStream_t st, Scratch* out) {
+  *out = Scratch::kKept;
+  if (st == ctx->stream) return PRISM_HIP_OK;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  HIP_TRY(ctx, hipStreamIsCapturing(st, &cap));
+  *out = cap == hipStreamCaptureStatusNone ? Scratch::kCall : Scratch::kNone;
+  return PRISM_HIP_OK;
+}
+
 int launch_gemm(prism_hip_ctx* ctx, const prism_hip_weight* w, const void* d_X, uint32_t M, void* d_Y,
                 hipStream_t st, float* fixed = nullptr) {
   if (!lookup_takes(ctx, w, d_X, M, false)) return launch_gemv_passes(ctx, w, nullptr, d_X, M, d_Y, st);
-  const bool lent = !fixed && st != ctx->stream;
-  return run_gemm(ctx, w, plan_gemm(w->bits, M, w->dim_m, w->dim_n, (uint32_t)ctx->num_cu, lent), d_X, M, d_Y, st, fixed);
+  Scratch sc = Scratch::kKept;  // (`fixed` is)
+  const int rc = fixed ? PRISM_HIP_OK : scratch_of(ctx, st, &sc);
+  if (rc) return rc;
+  return run_gemm(ctx, w, plan_gemm(w->bits, M, w->dim_m, w->dim_n, (uint32_t)ctx->num_cu, sc), d_X, M, d_Y, st, fixed);
 }
 
 // prism_hip_gemv and its like: several vectors may be the lookup GEMM's.
-// Under the capture of a caller's stream they take the form without scratch:
-// a captured GEMV is kernels alone, with no memory of its own in the graph.
 int launch_gemv(prism_hip_ctx* ctx, const prism_hip_weight* w, const prism_hip_weight* w2, const void* d_x,
                 uint32_t nb, void* d_y, hipStream_t st, void* d_y2 = nullptr) {
   if (w2 || !lookup_takes(ctx, w, d_x, nb, true)) return launch_gemv_passes(ctx, w, w2, d_x, nb, d_y, st, d_y2);
-  const bool lent = st != ctx->stream;
-  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  if (lent) HIP_TRY(ctx, hipStreamIsCapturing(st, &cap));
-  GemmPlan p;
-  if (cap == hipStreamCaptureStatusNone) {
-    p = plan_gemm(w->bits, nb, w->dim_m, w->dim_n, (uint32_t)ctx->num_cu, lent);
-  } else {
-    p.tt = nb > 32 ? 2 : 1;
-    plan_sizes(&p, w->bits, nb, w->dim_m, w->dim_n);
-  }
-  return run_gemm(ctx, w, p, d_x, nb, d_y, st, nullptr);
+  Scratch sc;
+  const int rc = scratch_of(ctx, st, &sc);
+  if (rc) return rc;
+  return run_gemm(ctx, w, plan_gemm(w->bits, nb, w->dim_m, w->dim_n, (uint32_t)ctx->num_cu, sc), d_x, nb, d_y, st,
+                  nullptr);
 }
 
 int launch_decode(prism_hip_ctx* ctx, const prism_hip_weight* w, uint32_t row0, uint32_t nrows, void* d_out,

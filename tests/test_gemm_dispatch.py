@@ -104,3 +104,14 @@ def test_noalloc_is_planned_without_a_price_for_scratch(bits, n, k):
     for row in fake_hip.call(__name__, "plans", bits, n, k, [24, 64, 96, 200, 300], ["own", "noalloc own", "noalloc lent"]):
         assert row["noalloc lent"]["kernels"] == row["noalloc own"]["kernels"] == row["own"]["kernels"]
         assert row["noalloc lent"]["memory"] == []
+
+
+@pytest.mark.parametrize("bits,n,k", [(4, 14336, 4096), (8, 14336, 4096), (4, 4096, 14336), (8, 1001, 1032), (4, 64, 8192)])
+def test_a_captured_call_is_kernels_alone(bits, n, k):
+    """Under the capture of a caller's stream nothing is allocated or freed, and
+    no kernel needs scratch."""
+    ms = [9, 16, 24, 33, 64, 96, 203, 256, 257, 300, 1024, 2048]
+    for row in fake_hip.call(__name__, "plans", bits, n, k, ms, ["capture", "gemv capture"]):
+        for how in row:
+            assert row[how]["memory"] == [] and row[how]["kernels"]
+            assert not [x for x in row[how]["kernels"] if "pack" in x[0] or "split_sum" in x[0]], row[how]
