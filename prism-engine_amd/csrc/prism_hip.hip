@@ -1315,18 +1315,14 @@ enum class Scratch { kKept, kCall, kNone };
 // The fastest plan by that estimate.  k_gemm_lookup_x up to 256 tokens (X
 // unpacked costs no launch: 14336 x 4096, 33 tokens 15 us; but 128 tokens 32
 // against 23.4), k_gemm_lookup above 64.  Scratch of the
-// call's own is allocated and freed on each call, about 22 us of host time.  4-bit calls of 49..64 tokens whose row blocks fit the CUs always
-// split K: tests/test_zz_no_alloc.py holds 64 tokens of 14336 x 4096 to a plan
-// with partials, though it is the slower one there (22.9 against 15.6 us
-// unsplit).
+// call's own is allocated and freed on each call, about 22 us of host time.
 GemmPlan plan_gemm(uint32_t bits, uint32_t M, uint32_t N, uint32_t K, uint32_t num_cu, Scratch scratch) {
   GemmPlan best;
   float best_us = 3.4e38f;
   // (weights that run_gemm cuts into row slabs have no partials)
   const uint32_t max_split = (uint64_t)N * K * bits / 8 < kMaxIndexBytes ? 16 : 1;
-  const uint32_t min_split = scratch != Scratch::kNone && bits == 4 && M > 48 && M <= 64 && N <= 64 * num_cu ? 2 : 1;
   auto consider = [&](bool packed, int rt, int tt, uint32_t ks) {
-    for (uint32_t split = min_split; split <= max_split; split *= 2) {
+    for (uint32_t split = 1; split <= max_split; split *= 2) {
       GemmPlan p;
       p.packed = packed;
       p.rt = rt;

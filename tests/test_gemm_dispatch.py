@@ -115,3 +115,14 @@ def test_a_captured_call_is_kernels_alone(bits, n, k):
         for how in row:
             assert row[how]["memory"] == [] and row[how]["kernels"]
             assert not [x for x in row[how]["kernels"] if "pack" in x[0] or "split_sum" in x[0]], row[how]
+
+
+@pytest.mark.parametrize("n,k", [(14336, 4096), (4864, 896), (6144, 4096)])
+def test_no_split_where_unsplit_is_faster(n, k):
+    """4-bit calls of 49..64 tokens on row blocks that fill a good part of the
+    CUs: K is not split (14336 x 4096 14.9 us against 22.4 in two splits, 4864
+    x 896 5.4 against 8.3), and so a caller's stream allocates nothing."""
+    for row in fake_hip.call(__name__, "plans", 4, n, k, [48, 49, 56, 64], ["own", "lent"]):
+        for how in row:
+            assert [x[0].split("<")[0] for x in row[how]["kernels"]] == ["k_gemm_lookup_x"], row[how]
+            assert row[how]["memory"] == []

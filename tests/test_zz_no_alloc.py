@@ -69,12 +69,12 @@ def test_gemm_noalloc_errors(pe, gpu_ctx):
 
 def test_gemm_noalloc_replayed_from_a_hip_graph(pe, gpu_ctx):
     """The no-alloc GEMM captured in a HIP graph: the split-K path (4-bit
-    14336 x 4096, M = 64: k_gemm_w4 in 4 K splits writing the static
+    4096 x 14336, M = 64: k_gemm_lookup_x in K splits writing the static
     scratch, then k_gemm_split_sum) makes no call that capture rejects, and
     every replay, each with new X copied in eagerly between replays,
     equals prism_hip_gemm_dev on the same X bit for bit."""
     import torch
-    N, K, M = 14336, 4096, 64
+    N, K, M = 4096, 14336, 64
     t = pe.synth_tensor(N, K, 4, seed=404)
     w = gpu_ctx.upload_tensor(t)
     s = torch.cuda.Stream()
