@@ -131,7 +131,7 @@ __device__ __forceinline__ void gwd_steps(uint32_t it, uint32_t nk, F& f, std::i
   ((it + I < nk ? (f(std::integral_constant<int, I>{}, it + I), 0) : 0), ...);
 }
 
-// MI = 32-row M subtiles per block (BM = 32 MI): 8, or 4 for more blocks.
+// MI = 32-row M subtiles per block (BM = 32 MI): 8, or 4 or 2 for fewer tokens and more blocks.
 // GI: the weights are in the GI layout with G rows per group (gemv_lpr.hpp;
 // lut and idx both point at it).  A K step's index bytes of a row are two
 // 16-byte chunks; DMA instruction i of wave w carries chunk i of its 64 rows
@@ -141,7 +141,7 @@ template <int MI, bool GI>
 __global__ __launch_bounds__(256) void k_gemm_w4(const uint8_t* __restrict__ lut, const uint8_t* __restrict__ idx,
                                                  const uint16_t* __restrict__ X, uint16_t* __restrict__ Y, uint32_t M,
                                                  uint32_t N, uint32_t K, uint32_t G) {
-  static_assert(MI == 4 || MI == 8, "32-row M subtiles per block");
+  static_assert(MI == 2 || MI == 4 || MI == 8, "32-row M subtiles per block");
   constexpr int BM = 32 * MI, BN = GW4_BN, BK = GW4_BK, S = gwd_stages<MI>();
   constexpr int XS = BM * BK / 8;     // 16-byte X slots per stage
   constexpr int SL = XS + GWD_WSLOTS;

@@ -1121,8 +1121,8 @@ int launch_gemv_passes(prism_hip_ctx* ctx, const prism_hip_weight* w, const pris
 // k_gemm_lookup_x (X as it is, tt x 32 tokens a workgroup) or k_gemm_lookup
 // (X packed first; rt x 32 rows and tt x 32 tokens a wave, ks waves sharing a
 // token group's K range), over `split` ranges of K whose fp32 partials
-// k_gemm_split_sum adds in order, `tokens` of X at a time; or k_gemm_w4 with
-// 32 * w4 tokens a block.
+// k_gemm_split_sum adds in order, `tokens` of X at a time; or, w4 = 2, 4 or 8,
+// k_gemm_w4 with 32 * w4 tokens a block.
 struct GemmPlan {
   int w4 = 0;
   bool packed = false;
@@ -1182,7 +1182,10 @@ int run_gemm_w4(prism_hip_ctx* ctx, const prism_hip_weight* w, int mi, const voi
   uint16_t* Y = static_cast<uint16_t*>(d_Y);
   uint32_t N = w->dim_m, K = w->dim_n, G = w->gi;
   const void* fn;
-  if (mi == 4)
+  if (mi == 2)
+    fn = G ? reinterpret_cast<const void*>(&prism::k_gemm_w4<2, true>)
+           : reinterpret_cast<const void*>(&prism::k_gemm_w4<2, false>);
+  else if (mi == 4)
     fn = G ? reinterpret_cast<const void*>(&prism::k_gemm_w4<4, true>)
            : reinterpret_cast<const void*>(&prism::k_gemm_w4<4, false>);
   else
@@ -1277,45 +1280,78 @@ int run_gemm(prism_hip_ctx* ctx, const prism_hip_weight* w, GemmPlan p, const vo
   return PRISM_HIP_OK;
 }
 
-// Estimated time of a plan in us on MI355X: whole rounds of workgroups over
-// the CUs, each a fixed part (LUT loads, tables, the sum over K slices, the
-// store) and the steps of one wave, plus the launches around it.  Fitted to
-// 14336 x 4096, 4096 x 14336, 4096 x 4096 and 1024 x 4096 at 8..2048 tokens;
-// measured times are within 30 % of it and the order of the candidates is
-// theirs but for near ties.
+// Estimated time of a plan in us on MI355X.  Fitted to every plan of 22 shapes
+// (64 x 4096 .. 151936 x 896) at 5..2048 tokens; the estimates are within 4..9 %
+// (root mean square) of the measured times, and the plan that they pick is on
+// average 1 % slower than the best one, at most 27 %.
 float gemm_plan_us(const GemmPlan& p, uint32_t bits, uint32_t M, uint32_t N, uint32_t K, uint32_t num_cu) {
-  // fixed us, us per step: k_gemm_lookup_x tt = 1, 2; k_gemm_lookup 64 x 64
-  // and 128 x 64 (4 bits) or 64 x 128 (8 bits)
-  static const float kFit[2][4][2] = {{{3.0f, 1.0f}, {5.0f, 1.2f}, {7.0f, 1.1f}, {12.0f, 1.55f}},
-                                      {{4.0f, 0.8f}, {4.5f, 0.95f}, {8.0f, 0.75f}, {12.0f, 1.05f}}};
-  const float* fit = kFit[bits == 8][p.packed ? (p.rt * p.tt > 4 ? 3 : 2) : p.tt - 1];
-  const uint32_t rows = p.packed ? 32u * p.rt : 64u;
+  // rounds of workgroups over the CUs: a last round that is not full counts half whole, half
+  // for its share of the CUs
+  auto rounds = [&](uint64_t groups) {
+    const float fill = (float)groups / (float)num_cu;
+    return 0.5f * std::max(1.0f, fill) + 0.5f * (float)((groups + num_cu - 1) / num_cu);
+  };
+  if (p.w4) {
+    // blocks of 64, 128 and 256 tokens: fixed us, us per step, more with all CUs busy; the same for
+    // each round after the first
+    static const float kW4[3][5] = {{3.85f, 0.67f, 0.16f, 2.4f, 0.65f}, {6.0f, 0.79f, 0.26f, 5.9f, 1.15f},
+                                    {8.1f, 1.18f, 0.48f, 6.7f, 1.98f}};
+    const float* f = kW4[p.w4 == 8 ? 2 : p.w4 / 4];
+    const uint64_t tiles = (uint64_t)((M + 32u * p.w4 - 1) / (32u * p.w4)) * ((N + prism::GW4_BN - 1) / prism::GW4_BN);
+    const float steps = (float)(K / prism::GW4_BK), busy = std::min(1.0f, (float)tiles / (float)num_cu);
+    return f[0] + steps * (f[1] + f[2] * busy) + (rounds(tiles) - 1.0f) * (f[3] + steps * f[4]);
+  }
+  const uint32_t rows = p.packed ? 32u * p.rt : 64u, blocks = (N + rows - 1) / rows;
   const uint32_t group = 32u * p.tt * (p.packed ? prism::kLkWaves / p.ks : 1u);
-  const uint64_t groups = (uint64_t)((N + rows - 1) / rows) * ((M + group - 1) / group) * p.split;
-  const uint32_t steps = (p.packed ? 2u : 1u) * ((p.per_split + p.ks - 1) / p.ks);
-  float us = (float)((groups + num_cu - 1) / num_cu) * (fit[0] + fit[1] * (float)steps);
-  if (p.packed) us += 2.5f + (float)M * (float)K * 1e-6f;                    // k_pack_x: 4 M K bytes
-  if (p.split > 1) us += 2.5f + (float)p.split * (float)M * (float)N * 1.8e-6f;  // the partials out and in
-  return us;
-}
-
-// The same for k_gemm_w4 (4 bits, blocks of 32 mi x 256), whose blocks slow
-// down as more CUs run them.
-float gemm_w4_us(int mi, uint32_t M, uint32_t N, uint32_t K, uint32_t num_cu) {
-  const uint32_t tiles = (M + 32u * mi - 1) / (32u * mi) * ((N + prism::GW4_BN - 1) / prism::GW4_BN);
-  const float busy = std::min(1.0f, (float)tiles / (float)num_cu);
-  const float step = mi == 8 ? 1.25f + 0.5f * busy : 0.45f + 0.74f * busy;
-  return (float)((tiles + num_cu - 1) / num_cu) * ((mi == 8 ? 6.5f : 8.5f) + step * (float)(K / prism::GW4_BK));
+  const uint64_t groups = (uint64_t)blocks * ((M + group - 1) / group) * p.split;
+  const float steps = (float)((p.packed ? 2u : 1u) * ((p.per_split + p.ks - 1) / p.ks));
+  // MB of x that the row blocks read, and of partials that go out
+  const float x_mb = (float)blocks * (float)M * (float)K * 2e-6f;
+  const float p_m = (float)p.split * (float)M * (float)N * 1e-6f;
+  if (!p.packed) {
+    // 32 and 64 tokens: fixed us (LUT loads, tables, sum, store), us per step; the same for each
+    // round after the first; us per MB of x; the sum's launch and its us per million partials
+    static const float kX[2][2][7] = {
+        {{4.15f, 0.64f, 2.2f, 0.74f, 0.03f, 1.9f, 1.7f}, {5.25f, 1.0f, 3.7f, 1.03f, 0.03f, 1.85f, 1.15f}},
+        {{4.55f, 0.545f, 2.95f, 0.68f, 0.05f, 2.2f, 1.55f}, {5.55f, 0.655f, 4.4f, 0.62f, 0.06f, 2.2f, 1.17f}}};
+    const float* f = kX[bits == 8][p.tt - 1];
+    return f[0] + steps * f[1] + (rounds(groups) - 1.0f) * (f[2] + steps * f[3]) + f[4] * x_mb +
+           (p.split > 1 ? f[5] + f[6] * p_m : 0.0f);
+  }
+  // 64 x 64 and 128 x 64 (4 bits) or 64 x 128 (8 bits) a wave: fixed us and us per step, more with
+  // all waves at work (not past M) and with each doubling of the waves on one token group, in whole
+  // rounds; us per MB of x; k_pack_x, a launch and its us per million elements; the sum as above
+  static const float kP[2][2][9] = {{{3.77f, 0.058f, 0.511f, 0.058f, 0.026f, 4.87f, 1.5f, 2.24f, 0.9f},
+                                     {7.78f, 0.108f, 0.62f, 0.058f, 0.059f, 4.42f, 1.34f, 1.87f, 0.87f}},
+                                    {{4.6f, 0.029f, 0.507f, 0.038f, 0.023f, 4.0f, 1.355f, 2.72f, 0.58f},
+                                     {8.86f, 0.113f, 0.616f, 0.033f, 0.02f, 4.08f, 1.31f, 2.39f, 0.64f}}};
+  const float* f = kP[bits == 8][p.rt * p.tt > 4];
+  const float live = std::min(1.0f, (float)(p.ks * ((M + 32u * p.tt - 1) / (32u * p.tt))) / (float)prism::kLkWaves);
+  const float doublings = p.ks == 8 ? 3.0f : p.ks == 4 ? 2.0f : p.ks == 2 ? 1.0f : 0.0f;
+  return (float)((groups + num_cu - 1) / num_cu) * (f[0] + steps * (f[1] + (f[2] + doublings * f[3]) * live)) +
+         f[4] * x_mb + f[5] + f[6] * (float)M * (float)K * 1e-6f + (p.split > 1 ? f[7] + f[8] * p_m : 0.0f);
 }
 
 // Where a call's scratch (packed X, partials) comes from: kept memory, the pool
 // for this call, or none may be used.
 enum class Scratch { kKept, kCall, kNone };
 
-// The fastest plan by that estimate.  k_gemm_lookup_x up to 256 tokens (X
-// unpacked costs no launch: 14336 x 4096, 33 tokens 15 us; but 128 tokens 32
-// against 23.4), k_gemm_lookup above 64.  Scratch of the
-// call's own is allocated and freed on each call, about 22 us of host time.
+// The fastest plan by that estimate.
+//  * k_gemm_lookup_x, to 256 tokens where there is another (X unpacked costs no
+//    launch, but is read again by each 64 rows: 14336 x 4096, 33 tokens 13.6 us
+//    against 20.5 packed, 128 tokens 29.5 against 22.8);
+//  * k_gemm_lookup above 64;
+//  * k_gemm_w4, which decodes each block's weights once, above 32: from half a
+//    block for each CU on (151936 x 896 at 64 / 128 / 256 tokens 34.7 / 58.8 /
+//    92.8 us against 65.3 / 85.7 / 112), and above 256 wherever the estimate
+//    says so (18944 x 3584, 768 tokens 98 against 113 us, 14336 x 4096, 1024
+//    tokens 113 against 115).
+// Of plans that the estimate cannot tell apart, the one in a single launch goes
+// first, then the lookup GEMM (4 and 7 %: 4096 x 14336, 203 tokens, 44.9 us
+// unpacked against 46.3; 14336 x 4096, 2048 tokens, 219 packed against 225).
+// Scratch of the call's own is allocated and freed on each call: 3..5 us more, and
+// no call below about 22 us of host time (14336 x 4096, 80 / 300 tokens 23.6 / 51.5
+// us with kept scratch, 28.6 / 54.4 with its own).
 GemmPlan plan_gemm(uint32_t bits, uint32_t M, uint32_t N, uint32_t K, uint32_t num_cu, Scratch scratch) {
   GemmPlan best;
   float best_us = 3.4e38f;
@@ -1332,7 +1368,8 @@ GemmPlan plan_gemm(uint32_t bits, uint32_t M, uint32_t N, uint32_t K, uint32_t n
       if (!plan_sizes(&p, bits, M, N, K)) continue;
       if (scratch == Scratch::kNone && p.x_bytes + p.p_bytes) continue;
       float us = gemm_plan_us(p, bits, M, N, K, num_cu);
-      if (scratch == Scratch::kCall && p.x_bytes + p.p_bytes) us = std::max(us, 22.0f);
+      if (p.x_bytes + p.p_bytes) us *= 1.04f;
+      if (scratch == Scratch::kCall && p.x_bytes + p.p_bytes) us = std::max(us + 4.0f, 22.0f);
       if (us < best_us) {
         best_us = us;
         best = p;
@@ -1340,7 +1377,7 @@ GemmPlan plan_gemm(uint32_t bits, uint32_t M, uint32_t N, uint32_t K, uint32_t n
     }
   };
   if (M <= 256 || scratch == Scratch::kNone) {
-    consider(false, 2, 1, prism::kLkWaves);
+    if (M <= 64) consider(false, 2, 1, prism::kLkWaves);
     if (M > 32) consider(false, 2, 2, prism::kLkWaves);
   }
   if (M > 64)
@@ -1351,18 +1388,17 @@ GemmPlan plan_gemm(uint32_t bits, uint32_t M, uint32_t N, uint32_t K, uint32_t n
       else
         consider(true, 2, 4, ks);
     }
-  // k_gemm_w4 decodes each block's weights once for 128 or 256 tokens: ahead
-  // where its blocks fill the CUs better (14336 x 4096, 768 tokens 100
-  // against 109 us, 18944 x 3584 103 against 114; 2048 tokens 228..237
-  // against 218..228, 4096 x 14336 at 1024 tokens 298 against 148)
-  if (bits == 4 && M > 256 && K % prism::GW4_BK == 0 && (uint64_t)N * (K / 2) < (1ull << 31) &&
+  if (bits == 4 && M > 32 && K % prism::GW4_BK == 0 && (uint64_t)N * (K / 2) < (1ull << 31) &&
       (uint64_t)K * 512 < (1ull << 31))
-    for (int mi = 4; mi <= 8; mi *= 2) {
-      const float us = gemm_w4_us(mi, M, N, K, num_cu);
+    for (int mi = 2; mi <= 8; mi *= 2) {
+      const uint64_t tiles = (uint64_t)((M + 32u * mi - 1) / (32u * mi)) * ((N + prism::GW4_BN - 1) / prism::GW4_BN);
+      if (M <= 256 && 2 * tiles < num_cu) continue;
+      GemmPlan p;
+      p.w4 = mi;
+      const float us = 1.07f * gemm_plan_us(p, bits, M, N, K, num_cu);
       if (us < best_us) {
         best_us = us;
-        best = GemmPlan{};
-        best.w4 = mi;
+        best = p;
       }
     }
   if (best_us > 3e38f) {  // rows too long for the scratch: the kernel that needs none

@@ -126,3 +126,28 @@ def test_no_split_where_unsplit_is_faster(n, k):
         for how in row:
             assert [x[0].split("<")[0] for x in row[how]["kernels"]] == ["k_gemm_lookup_x"], row[how]
             assert row[how]["memory"] == []
+
+
+def _names(row):
+    return [x[0].split("<")[0] for x in row["kernels"]]
+
+
+@pytest.mark.parametrize("n,k", [(151936, 896), (65536, 1024)])
+def test_tall_matrices_take_register_decode(n, k):
+    """An LM head over 33..256 tokens: blocks of k_gemm_w4 fill the CUs several
+    times over, where each 64 rows of the lookup GEMM build tables for 448
+    index bytes a row (151936 x 896, 64 tokens 34.7 against 65.3 us)."""
+    for row in fake_hip.call(__name__, "plans", 4, n, k, [33, 48, 64, 96, 128, 256], ["own", "lent", "capture"]):
+        for how in row:
+            assert _names(row[how]) == ["k_gemm_w4"], row[how]
+
+
+def test_the_plans_measured_fastest():
+    """The plans that were fastest, or within 1 % of it, when each was measured
+    (14336 x 4096 and 4096 x 14336, 4 bits), by kernel and tile."""
+    want = {(14336, 4096): {33: "k_gemm_lookup_x<4, 2", 64: "k_gemm_lookup_x<4, 2", 256: "k_gemm_lookup<4, 4, 2",
+                            512: "k_gemm_lookup<4, 4, 2", 2048: "k_gemm_lookup<4, 4, 2"},
+            (4096, 14336): {24: "k_gemm_lookup_x<4, 1", 203: "k_gemm_lookup_x<4, 2", 1024: "k_gemm_lookup<4, 4, 2"}}
+    for (n, k), kernels in want.items():
+        for (m, name), row in zip(kernels.items(), fake_hip.call(__name__, "plans", 4, n, k, list(kernels), ["own"])):
+            assert any(x[0].startswith(name) for x in row["own"]["kernels"]), (n, k, m, row)

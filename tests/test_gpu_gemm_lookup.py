@@ -23,7 +23,10 @@ CASES = [
     (4, 64, 64, 17, "x"), (4, 65, 72, 9, "x"), (4, 127, 1000, 33, "x"), (4, 130, 1096, 48, "x"),
     (4, 200, 2048, 49, "x"), (4, 63, 4096, 64, "x"), (4, 129, 128, 65, "x"), (4, 9100, 2048, 40, "x"),
     (4, 129, 136, 257, "p"), (4, 257, 1000, 300, "p"), (4, 1001, 1032, 513, "p"), (4, 3, 8, 270, "p"),
-    (4, 640, 648, 511, "p"), (4, 9100, 2112, 128, "p"), (4, 3584, 2048, 300, "p"), (4, 2000, 1024, 300, "w"),
+    (4, 640, 648, 511, "p"), (4, 9100, 2112, 230, "p"), (4, 3584, 2048, 300, "p"),
+    # k_gemm_w4 of 2, 4 and 8 token tiles, one K step and more, GI groups of 40
+    (4, 40000, 64, 64, "w"), (4, 33000, 128, 33, "w"), (4, 32900, 192, 129, "w"), (4, 32900, 192, 255, "w"),
+    (4, 16500, 512, 300, "w"), (4, 9100, 2112, 400, "w"),
     (8, 64, 32, 17, "x"), (8, 66, 40, 10, "x"), (8, 130, 1000, 33, "x"), (8, 200, 2048, 64, "x"), (8, 9100, 2048, 20, "x"),
     (8, 129, 64, 257, "p"), (8, 255, 72, 290, "p"), (8, 1001, 1032, 300, "p"), (8, 9100, 2048, 290, "p"),
     (8, 5, 8, 266, "p"),
@@ -37,7 +40,7 @@ def test_lookup_gemm_edges(pe, oracle, gpu_ctx, bits, N, K, M, kind):
     X = pe.synth_x(M, K, seed=M)
     Y = gpu_ctx.gemm(w, X)
     ran = gpu_ctx.last_kernels()
-    want = {"x": "k_gemm_lookup_x<", "p": "k_gemm_lookup<", "w": "k_gemm_"}[kind]
+    want = {"x": "k_gemm_lookup_x<", "p": "k_gemm_lookup<", "w": "k_gemm_w4<"}[kind]
     assert want in ran, ran
     _check(pe, Y, oracle.gemm(X, t.payload, N, K, bits, threads=8), f"{bits}-bit {M}x{N}x{K} ({ran})")
     w.free()
@@ -83,28 +86,34 @@ def test_lookup_gemm_ragged_rows_end(pe, oracle, gpu_ctx, bits, M):
     w.free()
 
 
-def test_lookup_gemm_scratch_over_streams(pe, oracle, gpu_ctx):
-    """Split and packed calls enqueued back to back on several streams and the
-    context's own, twice, with growing sizes, without a wait between them:
-    each output is its own."""
+def test_lookup_gemm_scratch_over_streams(pe, gpu_ctx):
+    """Packed calls and calls that split K, back to back on three streams and
+    the context's own, twice, without a wait between them: each output is, bit
+    for bit, that of the call made alone.  (All of them use scratch: packed X of
+    up to 8 MB, partials of up to 2 MB.)"""
     import torch
-    N, K = 200, 2048
-    t = pe.synth_tensor(N, K, 4, seed=77)
-    w = gpu_ctx.upload_tensor(t)
+    shapes = {"A": (14336, 4096), "B": (4096, 14336)}
+    w = {n: gpu_ctx.upload_tensor(pe.synth_tensor(*s, 4, seed=77)) for n, s in shapes.items()}
+    kinds = [("A", 203, "k_pack_x"), ("B", 24, "k_gemm_split_sum"), ("A", 256, "k_pack_x"), ("B", 300, "k_pack_x")]
     streams = [None] + [torch.cuda.Stream() for _ in range(3)]
     calls = []
     for rnd in range(2):
         for i, s in enumerate(streams):
-            M = 24 + 40 * ((i + rnd) % 4)
-            X = pe.synth_x(M, K, seed=100 * rnd + i)
-            calls.append((s, M, X, torch.from_numpy(X.view(np.int16)).cuda(), torch.empty((M, N), dtype=torch.int16, device="cuda")))
+            name, M, kernel = kinds[(i + rnd) % 4]
+            X = torch.from_numpy(pe.synth_x(M, shapes[name][1], seed=100 * rnd + i).view(np.int16)).cuda()
+            Y = torch.empty((2, M, shapes[name][0]), dtype=torch.int16, device="cuda")
+            torch.cuda.synchronize()
+            gpu_ctx.gemm_dev(w[name], X, M, Y[0], s)
+            assert kernel in gpu_ctx.last_kernels(), gpu_ctx.last_kernels()
+            torch.cuda.synchronize()
+            calls.append((s, w[name], X, M, Y))
+    for s, wt, X, M, Y in calls:
+        gpu_ctx.gemm_dev(wt, X, M, Y[1], s)
     torch.cuda.synchronize()
-    for s, M, _, dX, dY in calls:
-        gpu_ctx.gemm_dev(w, dX, M, dY, s)
-    torch.cuda.synchronize()
-    for _, M, X, _, dY in calls:
-        _check(pe, dY.cpu().numpy().view(np.uint16), oracle.gemm(X, t.payload, N, K, 4, threads=8), f"stream call M={M}")
-    w.free()
+    for i, (_, _, _, M, Y) in enumerate(calls):
+        assert torch.equal(Y[0], Y[1]), f"call {i} (M={M})"
+    for x in w.values():
+        x.free()
 
 
 def test_lookup_gemm_luts_past_2gib(pe, gpu_ctx):
