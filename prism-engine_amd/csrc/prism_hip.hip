@@ -1129,6 +1129,7 @@ struct GemmPlan {
   int rt = 2, tt = 1;
   uint32_t ks = prism::kLkWaves, split = 1, per_split = 0, tokens = 0;
   size_t x_bytes = 0, p_bytes = 0;  // scratch of one launch: packed X, partials
+  float us = 3.4e38f;               // its estimated time
 };
 
 // Grows the context stream's GEMM scratch.
@@ -1354,7 +1355,6 @@ enum class Scratch { kKept, kCall, kNone };
 // us with kept scratch, 28.6 / 54.4 with its own).
 GemmPlan plan_gemm(uint32_t bits, uint32_t M, uint32_t N, uint32_t K, uint32_t num_cu, Scratch scratch) {
   GemmPlan best;
-  float best_us = 3.4e38f;
   // (weights that run_gemm cuts into row slabs have no partials)
   const uint32_t max_split = (uint64_t)N * K * bits / 8 < kMaxIndexBytes ? 16 : 1;
   auto consider = [&](bool packed, int rt, int tt, uint32_t ks) {
@@ -1367,13 +1367,10 @@ GemmPlan plan_gemm(uint32_t bits, uint32_t M, uint32_t N, uint32_t K, uint32_t n
       p.split = split;
       if (!plan_sizes(&p, bits, M, N, K)) continue;
       if (scratch == Scratch::kNone && p.x_bytes + p.p_bytes) continue;
-      float us = gemm_plan_us(p, bits, M, N, K, num_cu);
-      if (p.x_bytes + p.p_bytes) us *= 1.04f;
-      if (scratch == Scratch::kCall && p.x_bytes + p.p_bytes) us = std::max(us + 4.0f, 22.0f);
-      if (us < best_us) {
-        best_us = us;
-        best = p;
-      }
+      p.us = gemm_plan_us(p, bits, M, N, K, num_cu);
+      if (p.x_bytes + p.p_bytes) p.us *= 1.04f;
+      if (scratch == Scratch::kCall && p.x_bytes + p.p_bytes) p.us = std::max(p.us + 4.0f, 22.0f);
+      if (p.us < best.us) best = p;
     }
   };
   if (M <= 256 || scratch == Scratch::kNone) {
@@ -1395,13 +1392,10 @@ GemmPlan plan_gemm(uint32_t bits, uint32_t M, uint32_t N, uint32_t K, uint32_t n
       if (M <= 256 && 2 * tiles < num_cu) continue;
       GemmPlan p;
       p.w4 = mi;
-      const float us = 1.07f * gemm_plan_us(p, bits, M, N, K, num_cu);
-      if (us < best_us) {
-        best_us = us;
-        best = p;
-      }
+      p.us = 1.07f * gemm_plan_us(p, bits, M, N, K, num_cu);
+      if (p.us < best.us) best = p;
     }
-  if (best_us > 3e38f) {  // rows too long for the scratch: the kernel that needs none
+  if (best.us > 3e38f) {  // rows too long for the scratch: the kernel that needs none
     best = GemmPlan{};
     best.tt = 2;
     plan_sizes(&best, bits, M, N, K);
@@ -1409,32 +1403,68 @@ GemmPlan plan_gemm(uint32_t bits, uint32_t M, uint32_t N, uint32_t K, uint32_t n
   return best;
 }
 
-// Whether M tokens go to the lookup GEMM rather than to GEMV passes (rows in
-// eights below 2^24, aligned x).  `gemv`: the GEMV entry points, whose GI calls of more
-// than 16 vectors stay with their passes.  MI355X, lookup against passes:
-//  * above 16 tokens always: two passes or more read the weights again
-//    (14336 x 4096, 32 tokens, 4 bits 10.9 against 24.7 us, 8 bits 19.9
-//    against 38.7; 151936 x 896, 24 tokens 52 against 72);
-//  * 9..16: where the matrix-core GEMV does not run (two tile passes: 2048 x
-//    2048, 16 tokens 6.9 against 12.0; 896 x 4864 7.8 against 12.6), and
-//    where it does, on rows of 4096 and more in one round of workgroups
-//    (14336 x 4096 9.9 against 12.3, 4096 x 14336 15.0 against 24.1; but
-//    18944 x 3584 17.9 against 16.0, 4864 x 896 5.2 against 4.6, 151936 x
-//    896 52 against 38);
-//  * 5..8: split-block rows of 8192 and more (4096 x 14336, 8 tokens, 4
-//    bits 14.5 against 19.3, 8 bits 23.6 against 29.8; at 4096 x 4096 8.5
-//    against 7.6), and tall 8-bit matrices on tile passes (10752 x 1056 8.0
-//    against 13.4).
-bool lookup_takes(const prism_hip_ctx* ctx, const prism_hip_weight* w, const void* d_x, uint32_t M, bool gemv) {
-  const uint32_t N = w->dim_m, K = w->dim_n;
+// Estimated time of M vectors (5..32; over GI weights 9 and more) as GEMV passes, us on MI355X:
+// the matrix-core GEMV in passes of 16 where it runs, fixed us, then for each
+// round of workgroups a fixed part and us per 1000 elements of K, with none and
+// with each vector; else the tile GEMV in passes of 8 vectors (fewer for long
+// rows), fixed us, more for each doubling of its vectors, and us per million
+// weights, with none and with each vector; no pass below the weights' bytes at 5.5
+// TB/s.  Fitted to the passes of the same 22 shapes, within 6..15 % (root mean
+// square).
+float passes_us(uint32_t bits, uint32_t gi, uint32_t M, uint32_t N, uint32_t K, uint32_t num_cu) {
+  const bool near = (uint64_t)N * K * bits / 8 < (1ull << 31);
+  const float floor_us = (float)N * ((float)K * (float)bits / 8 + (float)(2u << bits)) / 5.5e6f;  // the weights' bytes
+  float us = 0.0f;
+  if (gi || (K % prism::kGmGroup == 0 && N >= 4096 && near)) {
+    static const float kMfma[2][2][4] = {{{0.43f, 2.5f, 0.66f, 0.048f}, {0.3f, 3.6f, 1.35f, 0.05f}},
+                                         {{7.0f, 1.2f, 0.0f, 0.07f}, {0.0f, 17.0f, 0.0f, 0.08f}}};
+    const float* f = kMfma[gi != 0][bits == 8];
+    const float rounds = (float)(((N + 63) / 64 + num_cu - 1) / num_cu);
+    for (uint32_t n = M; n; n -= std::min(n, 16u))
+      us += std::max(floor_us, f[0] + rounds * (f[1] + (float)K * 1e-3f * (f[2] + f[3] * (float)std::min(n, 16u))));
+    return us;
+  }
+  static const float kTile[2][4] = {{2.8f, 0.47f, 0.078f, 0.032f}, {3.4f, 0.23f, 0.161f, 0.039f}};
+  const float* f = kTile[bits == 8];
+  const float mw = (float)N * (float)K * 1e-6f;
+  for (uint32_t n = M; n;) {
+    uint32_t c = std::min(n, 8u), nb, lg;
+    for (;; c = nb / 2) {  // vectors of a pass whose x fits the registers of 8 waves
+      for (nb = 1, lg = 0; nb < c; nb *= 2) lg++;
+      if (near && (K / 8 + 511) / 512 <= std::min(8u, 16 / nb)) break;
+      if (nb == 1) return 3.4e38f;  // the generic kernel, whatever it takes
+    }
+    us += std::max(floor_us, f[0] + f[1] * (float)lg + mw * (f[2] + f[3] * (float)nb));
+    n -= c;
+  }
+  return us;
+}
+
+// Whether M tokens can go to the GEMM kernels rather than to GEMV passes: 5 and
+// more, rows in eights below 2^24, aligned x.  GI calls of up to 8 vectors have
+// kernels of their own, and `gemv` (the GEMV entry points) keeps passes for those
+// of more than 16.
+bool gemm_can(const prism_hip_weight* w, const void* d_x, uint32_t M, bool gemv) {
+  const uint32_t K = w->dim_n;
   if (K % 8 != 0 || reinterpret_cast<uintptr_t>(d_x) % 16 != 0) return false;
   // 31-bit offsets: 64 tokens of x (and with that a tile's rows of indices) below 2 GiB
   if ((uint64_t)K * 64 * 2 >= (1ull << 31)) return false;
-  if (M > 16) return !(gemv && w->gi);
-  const bool mfma = K % prism::kGmGroup == 0 && (w->gi || N >= 4096);
-  if (M >= 9) return !mfma || (K >= 4096 && (N + 63) / 64 <= (uint32_t)ctx->num_cu);
-  if (M >= 5) return !w->gi && (K >= 8192 || (w->bits == 8 && !mfma && N >= 8192));
-  return false;
+  return w->gi ? M > 8 && !(gemv && M > 16) : M > 4;
+}
+
+// Whether the plan goes ahead of passes: above 32 tokens always, else by both
+// estimates, with 5 % for passes.  MI355X, plan against passes on the context's
+// stream: 14336 x 4096, 32 tokens, 4 bits 9.4 against 23.0 us, 16 tokens 9.2 against
+// 12.1; 4096 x 14336, 8 tokens 12.0 against 18.5, but 19.9 where it cannot split K
+// (a caller's stream, capture: 24.3); 4096 x 4096, 9 tokens 8.4 against 6.9; 256 x
+// 8192, 8 tokens 8.5 against 6.0, captured 15.8 against 7.1.  Up to 16 tokens the
+// matrix-core GEMV keeps what takes the lookup GEMM more than one round (18944 x
+// 3584, 12 tokens 13.7 against 16.0).
+bool gemm_goes_first(const prism_hip_ctx* ctx, const prism_hip_weight* w, uint32_t M, const GemmPlan& p) {
+  if (M > 32) return true;
+  const uint32_t N = w->dim_m, K = w->dim_n, num_cu = (uint32_t)ctx->num_cu;
+  if (M <= 16 && K % prism::kGmGroup == 0 && (N + 63) / 64 > num_cu) return false;
+  return 1.05f * p.us < passes_us(w->bits, w->gi, M, N, K, num_cu);
 }
 
 // A call on the context's stream uses its buffer, one on a caller's stream memory
@@ -1450,23 +1480,22 @@ int scratch_of(prism_hip_ctx* ctx, hipStream_t st, Scratch* out) {
 }
 
 int launch_gemm(prism_hip_ctx* ctx, const prism_hip_weight* w, const void* d_X, uint32_t M, void* d_Y,
-                hipStream_t st, float* fixed = nullptr) {
-  if (!lookup_takes(ctx, w, d_X, M, false)) return launch_gemv_passes(ctx, w, nullptr, d_X, M, d_Y, st);
-  Scratch sc = Scratch::kKept;  // (`fixed` is)
-  const int rc = fixed ? PRISM_HIP_OK : scratch_of(ctx, st, &sc);
-  if (rc) return rc;
-  return run_gemm(ctx, w, plan_gemm(w->bits, M, w->dim_m, w->dim_n, (uint32_t)ctx->num_cu, sc), d_X, M, d_Y, st, fixed);
+                hipStream_t st, float* fixed = nullptr, bool gemv = false) {
+  if (gemm_can(w, d_X, M, gemv)) {
+    Scratch sc = Scratch::kKept;  // (`fixed` is)
+    const int rc = fixed ? PRISM_HIP_OK : scratch_of(ctx, st, &sc);
+    if (rc) return rc;
+    const GemmPlan p = plan_gemm(w->bits, M, w->dim_m, w->dim_n, (uint32_t)ctx->num_cu, sc);
+    if (gemm_goes_first(ctx, w, M, p)) return run_gemm(ctx, w, p, d_X, M, d_Y, st, fixed);
+  }
+  return launch_gemv_passes(ctx, w, nullptr, d_X, M, d_Y, st);
 }
 
-// prism_hip_gemv and its like: several vectors may be the lookup GEMM's.
+// prism_hip_gemv and its like: several vectors may be the GEMM kernels'.
 int launch_gemv(prism_hip_ctx* ctx, const prism_hip_weight* w, const prism_hip_weight* w2, const void* d_x,
                 uint32_t nb, void* d_y, hipStream_t st, void* d_y2 = nullptr) {
-  if (w2 || !lookup_takes(ctx, w, d_x, nb, true)) return launch_gemv_passes(ctx, w, w2, d_x, nb, d_y, st, d_y2);
-  Scratch sc;
-  const int rc = scratch_of(ctx, st, &sc);
-  if (rc) return rc;
-  return run_gemm(ctx, w, plan_gemm(w->bits, nb, w->dim_m, w->dim_n, (uint32_t)ctx->num_cu, sc), d_x, nb, d_y, st,
-                  nullptr);
+  if (w2) return launch_gemv_passes(ctx, w, w2, d_x, nb, d_y, st, d_y2);
+  return launch_gemm(ctx, w, d_x, nb, d_y, st, nullptr, true);
 }
 
 int launch_decode(prism_hip_ctx* ctx, const prism_hip_weight* w, uint32_t row0, uint32_t nrows, void* d_out,

@@ -151,3 +151,48 @@ def test_the_plans_measured_fastest():
     for (n, k), kernels in want.items():
         for (m, name), row in zip(kernels.items(), fake_hip.call(__name__, "plans", 4, n, k, list(kernels), ["own"])):
             assert any(x[0].startswith(name) for x in row["own"]["kernels"]), (n, k, m, row)
+
+
+# (bits, N, K, vectors): those that GEMV passes take on a caller's stream and under capture, where K
+# is not split, and those that they take everywhere
+@pytest.mark.parametrize("bits,n,k,ms,own_too", [
+    (4, 256, 8192, [5, 6, 8], True), (4, 256, 8192, [9, 12, 16], False), (8, 256, 8192, [9, 16, 24], False),
+    (8, 512, 16384, [5, 8, 9, 12], False), (4, 4096, 4096, [9, 12], True), (8, 1024, 4096, [9, 12], False),
+    (4, 4096, 14336, [5, 8, 9], False), (8, 4864, 896, [9, 16], True), (4, 1024, 1024, [5, 8], True)])
+def test_passes_where_they_are_faster(bits, n, k, ms, own_too):
+    """Few rows of a long K, which the lookup GEMM needs its K splits for (256 x
+    8192, 8 bits, 8 vectors on a caller's stream 6.8 us in passes, 22.7 in the
+    lookup GEMM), and matrices that one pass of the matrix-core GEMV takes
+    (4096 x 4096, 9 vectors 6.9 us against 8.4)."""
+    hows = ["gemv lent", "gemv capture", "lent", "capture"] + (["own", "gemv own"] if own_too else [])
+    for row in fake_hip.call(__name__, "plans", bits, n, k, ms, hows):
+        for how in row:
+            assert all(x.startswith("k_gemv_") for x in _names(row[how])) and row[how]["memory"] == [], (how, row[how])
+
+
+@pytest.mark.parametrize("bits,n,k,ms", [(4, 14336, 4096, [9, 16]), (8, 14336, 4096, [9, 16]), (4, 2048, 2048, [9, 16, 24]),
+                                         (4, 896, 4864, [16, 24, 32]), (8, 10752, 1056, [8, 16]), (4, 151936, 896, [17, 32])])
+def test_the_lookup_gemm_where_it_is_faster(bits, n, k, ms):
+    """The other side: one round of row blocks, several tile passes, two passes
+    of the matrix-core GEMV; on every stream alike."""
+    for row in fake_hip.call(__name__, "plans", bits, n, k, ms, ["own", "lent", "capture"]):
+        for how in row:
+            assert _names(row[how])[0] == "k_gemm_lookup_x", (how, row[how])
+
+
+def without_memory(hip, pe, n, k, m, stream):
+    ctx = pe.Context(0)
+    w = ctx.upload_dev(fake_hip.Tensor(hip, payload_bytes(n, k, 4)), n, k, 4)
+    x, y = fake_hip.Tensor(hip, m * k * 2), fake_hip.Tensor(hip, m * n * 2)
+    hip.lib.fake_refuse(1)
+    hip.clear()
+    ctx.gemm_dev(w, x, m, y, stream)
+    return [[ln.name, ln.lk.P if ln.lk else 0] for ln in hip.launches]
+
+
+@pytest.mark.parametrize("stream", [None, STREAM])
+@pytest.mark.parametrize("n,k,m", [(4096, 14336, 24), (14336, 4096, 300)])
+def test_no_memory_for_scratch(n, k, m, stream):
+    """A plan whose scratch cannot be had (K split; X packed): the kernel that needs none."""
+    launched = fake_hip.call(__name__, "without_memory", n, k, m, stream)
+    assert len(launched) == 1 and "k_gemm_lookup_x" in launched[0][0] and not launched[0][1]

@@ -46,7 +46,7 @@ def test_lookup_gemm_edges(pe, oracle, gpu_ctx, bits, N, K, M, kind):
     w.free()
 
 
-@pytest.mark.parametrize("bits,batch,N,K", [(4, 12, 300, 1032), (4, 7, 100, 8200), (4, 16, 9000, 4096), (8, 6, 8200, 1064),
+@pytest.mark.parametrize("bits,batch,N,K", [(4, 12, 300, 1032), (4, 7, 100, 16392), (4, 16, 9000, 4096), (8, 6, 8200, 1064),
                                             (8, 24, 70, 264)])
 def test_lookup_gemv_batches(pe, oracle, gpu_ctx, bits, batch, N, K):
     """GEMV batches that the lookup GEMM takes."""
@@ -143,13 +143,12 @@ def test_lookup_gemm_luts_past_2gib(pe, gpu_ctx):
     w.free()
 
 
-@pytest.mark.parametrize("batch", [8, 40])
-def test_lookup_gemv_captured(pe, oracle, gpu_ctx, batch):
+@pytest.mark.parametrize("batch,N,K", [(12, 300, 1032), (40, 256, 8192)])
+def test_lookup_gemv_captured(pe, oracle, gpu_ctx, batch, N, K):
     """A GEMV of several vectors captured on the caller's stream: kernels alone,
     no K splits and no memory, and every replay takes the x that is there then,
-    with eager calls (which split K) between the replays."""
+    with eager calls (which split K at 8192) between the replays."""
     import torch
-    N, K = 256, 8192
     t = pe.synth_tensor(N, K, 4, seed=9)
     w = gpu_ctx.upload_tensor(t)
     dX = torch.zeros((batch, K), dtype=torch.int16, device="cuda")
