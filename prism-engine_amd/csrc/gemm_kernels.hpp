@@ -1,7 +1,8 @@
-// gemm_kernels.hpp -- palettized prefill GEMM for gfx950 (MFMA fp16 -> fp32)
-// with the weights decoded in registers, and the sum of split-K partials.
+// gemm_kernels.hpp -- palettized prefill GEMMs for gfx950 (MFMA fp16 -> fp32)
+// with the weights decoded in registers (4 bits) or through an LDS tile (8
+// bits), and the sum of split-K partials.
 //
-// Y[M x N] = X[M x K] . W^T with W[N x K] 4-bit palettized, fp32
+// Y[M x N] = X[M x K] . W^T with W[N x K] palettized, fp32
 // accumulation and fp16 (RNE) output: M independent lut_gemv_cpu rows
 // (compute-core/src/lut/evaluator.rs:21-44); the reference's own GEMM
 // template (templates/palettized_gemm.metal) is never dispatched.
@@ -341,6 +342,171 @@ __global__ __launch_bounds__(256) void k_gemm_w4(const uint8_t* __restrict__ lut
         if (m < M && n < N) yc[(size_t)m * N] = __builtin_bit_cast(uint16_t, (_Float16)acc[i][s][e]);
       }
   }
+}
+
+// ---------------------------------------------------------------------------
+// k_gemm8: 8-bit prefill GEMM without scratch, for captured calls of more than
+// a few hundred tokens (k_gemm_lookup_x reads X again for each 64 rows: 14336 x
+// 4096, 2048 tokens 577 us against 441; packed X in k_gemm_lookup, which needs
+// scratch, 263).  The block's 128 row LUTs stay in LDS; each 64-wide K step's
+// index tile is decoded through them into an fp16 B tile (256 (M) x 128 (N)
+// blocks), so that a decoded weight feeds 256 tokens.
+//  * 4 waves as 2 (M) x 2 (N): wave (wm, wn) owns rows [128 wm, +128) x
+//    columns [64 wn, +64) = 4 x 2 v_mfma_f32_32x32x16_f16 tiles.
+//  * LDS: LUTs 64 KB, X tile 256 x 64 and B tile 128 x 64 fp16 with a
+//    144-byte row pitch (16 rows at one 16-byte column land in 16 distinct
+//    4-bank groups).
+//  * The next step's global loads are issued before the current step's
+//    MFMAs; blocks are mapped XCD-aware like k_gemm_w4's.
+// Bound by the decode and two barriers a step: 1.6 us a step and round of blocks.
+// Requires K % 64 == 0 and 16-byte aligned X.
+constexpr int GM8_BM = 256;
+constexpr int GM8_BN = 128;
+constexpr int GM8_BK = 64;
+
+// GI: the weights are in the GI layout with G rows per group (gemv_lpr.hpp;
+// lut and idx both point at it); a thread's 16 index bytes of a K step are
+// one chunk of its row.
+template <bool GI>
+__global__ __launch_bounds__(256) void k_gemm8(const uint8_t* __restrict__ lut, const uint8_t* __restrict__ idx,
+                                               const uint16_t* __restrict__ X, uint16_t* __restrict__ Y, uint32_t M,
+                                               uint32_t N, uint32_t K, uint32_t G) {
+  constexpr int BM = GM8_BM, BN = GM8_BN, BK = GM8_BK, P = BK + 8;
+  constexpr int XU = BM * BK / 8 / 256;  // 16-byte X chunks per thread per step (8)
+  constexpr int WU = BN * BK / 16 / 256; // 16-byte index chunks per thread per step (2)
+  __shared__ __attribute__((aligned(16))) uint16_t sA[BM * P];
+  __shared__ __attribute__((aligned(16))) uint16_t sB[BN * P];
+  __shared__ __attribute__((aligned(16))) uint16_t sL[BN * 256];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = tid >> 6;
+  const int wm = wave >> 1, wn = wave & 1;
+
+  const uint32_t mt = (M + BM - 1) / BM;
+  const uint32_t nt = (N + BN - 1) / BN;
+  const uint32_t ntiles = mt * nt;
+  uint32_t t = blockIdx.x;
+  {
+    const uint32_t per = ntiles / 8, rem = ntiles % 8;
+    const uint32_t xcd = t % 8, slot = t / 8;
+    t = xcd * per + (xcd < rem ? xcd : rem) + slot;
+  }
+  const uint32_t n0 = (t % nt) * BN;
+  const uint32_t m0 = (t / nt) * BM;
+
+  // ---- LUTs of this block's rows -> LDS (rows past N are zero)
+  {
+    constexpr int U4 = BN * 256 * 2 / 16;
+    uint4* dst = reinterpret_cast<uint4*>(sL);
+    const uint32_t live_u4 = (N - n0 < (uint32_t)BN ? N - n0 : (uint32_t)BN) * 32;
+    for (int i = tid; i < U4; i += 256) {
+      // piece i % 32 of row n0 + i / 32 (GI: the block's rows may span groups)
+      const uint32_t r = n0 + (uint32_t)i / 32;
+      const uint4* src =
+          reinterpret_cast<const uint4*>(lut + (GI ? gi_lut_offset(G, r, K, 8) : (size_t)r * 512) + 16 * (i % 32));
+      dst[i] = (uint32_t)i < live_u4 ? *src : make_uint4(0, 0, 0, 0);
+    }
+  }
+
+  // chunk c = tid + 256 i: X row c / 8, column chunk c % 8; index row c / 4, chunk c % 4
+  uint4 ra[XU], rb[WU];
+  // GI: byte offset of chunk 0 of each of the thread's index rows
+  size_t wrow[WU];
+#pragma unroll
+  for (int i = 0; i < WU; i++) {
+    const uint32_t n = n0 + ((tid + 256 * i) >> 2);
+    wrow[i] = GI ? gi_chunk_offset(G, n < N ? n : 0u, 0, K, 8) : (size_t)n * K;
+  }
+  auto gload = [&](uint32_t k0) {
+#pragma unroll
+    for (int i = 0; i < XU; i++) {
+      const int c = tid + 256 * i;
+      const uint32_t m = m0 + (c >> 3);
+      ra[i] = (m < M) ? *reinterpret_cast<const uint4*>(X + (size_t)m * K + k0 + 8 * (c & 7)) : make_uint4(0, 0, 0, 0);
+    }
+#pragma unroll
+    for (int i = 0; i < WU; i++) {
+      const int c = tid + 256 * i;
+      const uint32_t n = n0 + (c >> 2);
+      const size_t off = GI ? wrow[i] + (size_t)(k0 / 16 + (c & 3)) * G * 16 : wrow[i] + k0 + 16 * (c & 3);
+      rb[i] = (n < N) ? *reinterpret_cast<const uint4*>(idx + off) : make_uint4(0, 0, 0, 0);
+    }
+  };
+  auto lstore = [&]() {
+#pragma unroll
+    for (int i = 0; i < XU; i++) {
+      const int c = tid + 256 * i;
+      *reinterpret_cast<uint4*>(&sA[(c >> 3) * P + 8 * (c & 7)]) = ra[i];
+    }
+#pragma unroll
+    for (int i = 0; i < WU; i++) {
+      const int c = tid + 256 * i, r = c >> 2;
+      const uint16_t* tb = &sL[r * 256];
+      const uint32_t w4[4] = {rb[i].x, rb[i].y, rb[i].z, rb[i].w};
+      uint32_t o[8];
+#pragma unroll
+      for (int q = 0; q < 4; q++)
+#pragma unroll
+        for (int p = 0; p < 2; p++) {
+          const uint32_t lo = tb[(w4[q] >> (16 * p)) & 255u];
+          const uint32_t hi = tb[(w4[q] >> (16 * p + 8)) & 255u];
+          o[2 * q + p] = lo | (hi << 16);
+        }
+      uint4* d = reinterpret_cast<uint4*>(&sB[r * P + 16 * (c & 3)]);
+      d[0] = make_uint4(o[0], o[1], o[2], o[3]);
+      d[1] = make_uint4(o[4], o[5], o[6], o[7]);
+    }
+  };
+
+  floatx16 acc[4][2];
+#pragma unroll
+  for (int i = 0; i < 4; i++)
+#pragma unroll
+    for (int j = 0; j < 2; j++)
+#pragma unroll
+      for (int e = 0; e < 16; e++) acc[i][j][e] = 0.0f;
+
+  const uint32_t nk = K / BK;
+  gload(0);
+  __syncthreads();  // sL ready
+  for (uint32_t ks = 0; ks < nk; ks++) {
+    lstore();
+    __syncthreads();
+    if (ks + 1 < nk) gload((ks + 1) * BK);
+#pragma unroll
+    for (int kk = 0; kk < BK; kk += 16) {
+      half8_t af[4], bf[2];
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const int r = wm * 128 + i * 32 + (lane & 31);
+        af[i] = *reinterpret_cast<const half8_t*>(&sA[r * P + kk + 8 * (lane >> 5)]);
+      }
+#pragma unroll
+      for (int j = 0; j < 2; j++) {
+        const int r = wn * 64 + j * 32 + (lane & 31);
+        bf[j] = *reinterpret_cast<const half8_t*>(&sB[r * P + kk + 8 * (lane >> 5)]);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i], bf[j], acc[i][j], 0, 0, 0);
+    }
+    __syncthreads();
+  }
+
+  // ---- epilogue: D lane layout: col = lane%32, row = 8*(e/4) + 4*(lane/32) + e%4
+#pragma unroll
+  for (int i = 0; i < 4; i++)
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+      const uint32_t n = n0 + wn * 64 + j * 32 + (lane & 31);
+#pragma unroll
+      for (int e = 0; e < 16; e++) {
+        const uint32_t m = m0 + wm * 128 + i * 32 + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
+        if (m < M && n < N) Y[(size_t)m * N + n] = __builtin_bit_cast(uint16_t, (_Float16)acc[i][j][e]);
+      }
+    }
 }
 
 // Y[i] = f16(P[0][i] + P[1][i] + ... + P[S-1][i]) over mn = M N elements,

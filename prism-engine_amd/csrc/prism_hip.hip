@@ -1122,9 +1122,10 @@ int launch_gemv_passes(prism_hip_ctx* ctx, const prism_hip_weight* w, const pris
 // (X packed first; rt x 32 rows and tt x 32 tokens a wave, ks waves sharing a
 // token group's K range), over `split` ranges of K whose fp32 partials
 // k_gemm_split_sum adds in order, `tokens` of X at a time; or, w4 = 2, 4 or 8,
-// k_gemm_w4 with 32 * w4 tokens a block.
+// k_gemm_w4 with 32 * w4 tokens a block, or, w8, k_gemm8.
 struct GemmPlan {
   int w4 = 0;
+  bool w8 = false;
   bool packed = false;
   int rt = 2, tt = 1;
   uint32_t ks = prism::kLkWaves, split = 1, per_split = 0, tokens = 0;
@@ -1176,31 +1177,29 @@ bool plan_sizes(GemmPlan* p, uint32_t bits, uint32_t M, uint32_t N, uint32_t K) 
 // Index (or LUT) bytes one launch addresses with 31-bit buffer offsets.
 constexpr size_t kMaxIndexBytes = 0x7F000000;
 
-int run_gemm_w4(prism_hip_ctx* ctx, const prism_hip_weight* w, int mi, const void* d_X, uint32_t M, void* d_Y,
-                hipStream_t st) {
+int run_gemm_blocks(prism_hip_ctx* ctx, const prism_hip_weight* w, const GemmPlan& p, const void* d_X, uint32_t M,
+                    void* d_Y, hipStream_t st) {
   const uint8_t *lut = w->lut(), *idx = w->idx();
   const uint16_t* X = static_cast<const uint16_t*>(d_X);
   uint16_t* Y = static_cast<uint16_t*>(d_Y);
   uint32_t N = w->dim_m, K = w->dim_n, G = w->gi;
   const void* fn;
-  if (mi == 2)
-    fn = G ? reinterpret_cast<const void*>(&prism::k_gemm_w4<2, true>)
-           : reinterpret_cast<const void*>(&prism::k_gemm_w4<2, false>);
-  else if (mi == 4)
-    fn = G ? reinterpret_cast<const void*>(&prism::k_gemm_w4<4, true>)
-           : reinterpret_cast<const void*>(&prism::k_gemm_w4<4, false>);
+#define PRISM_GI(K_, ...) \
+  (G ? reinterpret_cast<const void*>(&prism::K_<__VA_ARGS__ true>) : reinterpret_cast<const void*>(&prism::K_<__VA_ARGS__ false>))
+  if (p.w8)
+    fn = PRISM_GI(k_gemm8, );
   else
-    fn = G ? reinterpret_cast<const void*>(&prism::k_gemm_w4<8, true>)
-           : reinterpret_cast<const void*>(&prism::k_gemm_w4<8, false>);
+    fn = p.w4 == 2 ? PRISM_GI(k_gemm_w4, 2, ) : p.w4 == 4 ? PRISM_GI(k_gemm_w4, 4, ) : PRISM_GI(k_gemm_w4, 8, );
+#undef PRISM_GI
+  const uint32_t bm = p.w8 ? prism::GM8_BM : 32u * p.w4, bn = p.w8 ? prism::GM8_BN : prism::GW4_BN;
   void* args[] = {&lut, &idx, &X, &Y, &M, &N, &K, &G};
-  const uint32_t tiles = (M + 32u * mi - 1) / (32u * mi) * ((N + prism::GW4_BN - 1) / prism::GW4_BN);
-  HIP_TRY(ctx, launch_fn(fn, dim3(tiles), dim3(256), args, 0, st));
+  HIP_TRY(ctx, launch_fn(fn, dim3((M + bm - 1) / bm * ((N + bn - 1) / bn)), dim3(256), args, 0, st));
   return PRISM_HIP_OK;
 }
 
 int run_gemm(prism_hip_ctx* ctx, const prism_hip_weight* w, GemmPlan p, const void* d_X, uint32_t M, void* d_Y,
              hipStream_t st, float* fixed) {
-  if (p.w4) return run_gemm_w4(ctx, w, p.w4, d_X, M, d_Y, st);
+  if (p.w4 || p.w8) return run_gemm_blocks(ctx, w, p, d_X, M, d_Y, st);
   const uint32_t N = w->dim_m, K = w->dim_n, bits = w->bits, step = prism::lk_step(bits);
   const size_t need = p.x_bytes + p.p_bytes;
   // scratch: the caller's, the context stream's kept one, or on another
@@ -1292,6 +1291,10 @@ float gemm_plan_us(const GemmPlan& p, uint32_t bits, uint32_t M, uint32_t N, uin
     const float fill = (float)groups / (float)num_cu;
     return 0.5f * std::max(1.0f, fill) + 0.5f * (float)((groups + num_cu - 1) / num_cu);
   };
+  if (p.w8) {
+    const uint64_t tiles = (uint64_t)((M + prism::GM8_BM - 1) / prism::GM8_BM) * ((N + prism::GM8_BN - 1) / prism::GM8_BN);
+    return (float)((tiles + num_cu - 1) / num_cu) * (10.0f + 1.6f * (float)(K / prism::GM8_BK));
+  }
   if (p.w4) {
     // blocks of 64, 128 and 256 tokens: fixed us, us per step, more with all CUs busy; the same for
     // each round after the first
@@ -1347,6 +1350,9 @@ enum class Scratch { kKept, kCall, kNone };
 //    92.8 us against 65.3 / 85.7 / 112), and above 256 wherever the estimate
 //    says so (18944 x 3584, 768 tokens 98 against 113 us, 14336 x 4096, 1024
 //    tokens 113 against 115).
+//  * k_gemm8 where no scratch may be used, above 256 tokens at 8 bits (14336 x
+//    4096, 2048 tokens 441 us against 577 in k_gemm_lookup_x, 300 tokens 112
+//    against 85).
 // Of plans that the estimate cannot tell apart, the one in a single launch goes
 // first, then the lookup GEMM (4 and 7 %: 4096 x 14336, 203 tokens, 44.9 us
 // unpacked against 46.3; 14336 x 4096, 2048 tokens, 219 packed against 225).
@@ -1395,6 +1401,12 @@ GemmPlan plan_gemm(uint32_t bits, uint32_t M, uint32_t N, uint32_t K, uint32_t n
       p.us = 1.07f * gemm_plan_us(p, bits, M, N, K, num_cu);
       if (p.us < best.us) best = p;
     }
+  if (bits == 8 && scratch == Scratch::kNone && M > 256 && K % prism::GM8_BK == 0) {
+    GemmPlan p;
+    p.w8 = true;
+    p.us = gemm_plan_us(p, bits, M, N, K, num_cu);
+    if (p.us < best.us) best = p;
+  }
   if (best.us > 3e38f) {  // rows too long for the scratch: the kernel that needs none
     best = GemmPlan{};
     best.tt = 2;

@@ -196,3 +196,13 @@ def test_no_memory_for_scratch(n, k, m, stream):
     """A plan whose scratch cannot be had (K split; X packed): the kernel that needs none."""
     launched = fake_hip.call(__name__, "without_memory", n, k, m, stream)
     assert len(launched) == 1 and "k_gemm_lookup_x" in launched[0][0] and not launched[0][1]
+
+
+@pytest.mark.parametrize("n,k,m,kernel", [(14336, 4096, 512, "k_gemm8"), (14336, 4096, 2048, "k_gemm8"), (14336, 4096, 300, "k_gemm_lookup_x"),
+                                          (4096, 4096, 2048, "k_gemm8"), (4096, 4096, 512, "k_gemm_lookup_x"), (151936, 896, 512, "k_gemm8"),
+                                          (1001, 1032, 2048, "k_gemm_lookup_x")])
+def test_captured_8_bit_prefills(n, k, m, kernel):
+    """The kernel without scratch that each was measured fastest on (14336 x
+    4096, 2048 tokens 441 us against 577); K % 64 != 0 has one only."""
+    for row in fake_hip.call(__name__, "plans", 8, n, k, [m], ["capture"]):
+        assert _names(row["capture"]) == [kernel]

@@ -170,3 +170,42 @@ def test_lookup_gemv_captured(pe, oracle, gpu_ctx, batch, N, K):
         _check(pe, dY.cpu().numpy().view(np.uint16), ref, f"replay {i}")
         _check(pe, gpu_ctx.gemv(w, X), ref, f"eager {i}")
     w.free()
+
+
+# 8 bits, more than 256 tokens: k_gemm8 over GI groups of 40 and over split-block rows, tokens and rows
+# that do not fill its 256 x 128 blocks; the unpacked lookup GEMM where that is ahead; 4 bits
+@pytest.mark.parametrize("bits,N,K,M,kernel", [(8, 9100, 2048, 520, "k_gemm8<true>"), (8, 8200, 704, 600, "k_gemm8<false>"),
+                                               (8, 1001, 1032, 300, "k_gemm_lookup_x<8, 2"), (8, 200, 2048, 70, "k_gemm_lookup_x<8, 2"),
+                                               (4, 16500, 512, 300, "k_gemm_w4<4"), (4, 1001, 1032, 270, "k_gemm_lookup_x<4, 2")])
+def test_gemm_captured(pe, oracle, gpu_ctx, bits, N, K, M, kernel):
+    """gemm_dev captured on the caller's stream: one kernel and no memory; every
+    replay takes the X that is there then, with eager calls (which pack X)
+    between the replays.  Tokens at the edges of the blocks against the oracle."""
+    import torch
+    t = pe.synth_tensor(N, K, bits, seed=N)
+    w = gpu_ctx.upload_tensor(t)
+    dX = torch.zeros((M, K), dtype=torch.int16, device="cuda")
+    dY = torch.empty((M, N), dtype=torch.int16, device="cuda")
+    s = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        gpu_ctx.gemm_dev(w, dX, M, dY, s)
+    ran = gpu_ctx.last_kernels()
+    assert ran.startswith(kernel) and "+" not in ran, ran
+    rows = sorted({0, 1, 31, 32, 63, 64, 65, 127, 128, 255, 256, 257, 511, 512, M // 2, M - 2, M - 1} & set(range(M)))
+    for i in range(3):
+        X = pe.synth_x(M, K, seed=70 + i)
+        dX.copy_(torch.from_numpy(X.view(np.int16)))
+        dY.fill_(-1)
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        ref = oracle.gemm(np.ascontiguousarray(X[rows]), t.payload, N, K, bits, threads=8)
+        Y = dY.cpu().numpy().view(np.uint16)
+        _check(pe, Y[rows], ref, f"replay {i} ({ran})")
+        eager = gpu_ctx.gemm(w, X)
+        _check(pe, Y, eager, f"replay {i} against eager")
+        _check(pe, eager[rows], ref, f"eager {i}")
+    del g
+    w.free()
