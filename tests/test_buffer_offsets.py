@@ -752,7 +752,7 @@ def check_gemm_launches(launches, bits, M, N):
     return seen
 
 
-LK_CALLS = [(M, how) for M in (9, 33, 64, 65, 203, 512, 1030) for how in ("own", "lent", "capture", "noalloc")]
+LK_CALLS = [(M, how) for M in (9, 24, 33, 64, 65, 203, 512, 1030) for how in ("own", "lent", "capture", "noalloc")]
 
 
 # GI (both widths; 24-row tail groups), split-block, ragged K at both widths, few rows, long rows, an LM head
