@@ -1280,82 +1280,86 @@ int run_gemm(prism_hip_ctx* ctx, const prism_hip_weight* w, GemmPlan p, const vo
   return PRISM_HIP_OK;
 }
 
-// Estimated time of a plan in us on MI355X.  Fitted to every plan of 22 shapes
-// (64 x 4096 .. 151936 x 896) at 5..2048 tokens; the estimates are within 4..9 %
-// (root mean square) of the measured times, and the plan that they pick is on
-// average 1 % slower than the best one, at most 27 %.
+// Estimated time of a plan in us on MI355X.  Fitted to every plan of 580 shapes
+// (64 .. 151936 rows of 768 .. 16384, odd ones among them) at 5 to 11 numbers of
+// tokens each from 5 to 2048, for the least time lost by the plan it picks: with
+// scratch 0.5 % over the fastest plan on average, one in twenty over 4 %, at most 19;
+// without, 0.1 % and at most 24.  (Shapes left out of the fit: 0.6 and 0.1 %, at most
+// 17 and 14.)
 float gemm_plan_us(const GemmPlan& p, uint32_t bits, uint32_t M, uint32_t N, uint32_t K, uint32_t num_cu) {
-  // rounds of workgroups over the CUs: a last round that is not full counts half whole, half
-  // for its share of the CUs
-  auto rounds = [&](uint64_t groups) {
-    const float fill = (float)groups / (float)num_cu;
-    return 0.5f * std::max(1.0f, fill) + 0.5f * (float)((groups + num_cu - 1) / num_cu);
-  };
-  if (p.w8) {
-    const uint64_t tiles = (uint64_t)((M + prism::GM8_BM - 1) / prism::GM8_BM) * ((N + prism::GM8_BN - 1) / prism::GM8_BN);
-    return (float)((tiles + num_cu - 1) / num_cu) * (10.0f + 1.6f * (float)(K / prism::GM8_BK));
-  }
-  if (p.w4) {
-    // blocks of 64, 128 and 256 tokens: fixed us, us per step, more with all CUs busy; the same for
-    // each round after the first
-    static const float kW4[3][5] = {{3.85f, 0.67f, 0.16f, 2.4f, 0.65f}, {6.0f, 0.79f, 0.26f, 5.9f, 1.15f},
-                                    {8.1f, 1.18f, 0.48f, 6.7f, 1.98f}};
-    const float* f = kW4[p.w4 == 8 ? 2 : p.w4 / 4];
-    const uint64_t tiles = (uint64_t)((M + 32u * p.w4 - 1) / (32u * p.w4)) * ((N + prism::GW4_BN - 1) / prism::GW4_BN);
-    const float steps = (float)(K / prism::GW4_BK), busy = std::min(1.0f, (float)tiles / (float)num_cu);
-    return f[0] + steps * (f[1] + f[2] * busy) + (rounds(tiles) - 1.0f) * (f[3] + steps * f[4]);
+  const float mn = (float)M * (float)N * 1e-6f;
+  auto rounds = [&](uint64_t groups) { return (float)((groups + num_cu - 1) / num_cu); };  // over the CUs
+  if (p.w4 || p.w8) {
+    // k_gemm_w4 of 64, 128 and 256 tokens, k_gemm8: fixed us, us per step, more with all CUs busy; the
+    // same for each round after the first, of which a last one that is not full counts a quarter for
+    // its share of the CUs; us per million outputs
+    static const float kBlocks[4][6] = {{4.63f, 0.681f, 0.0327f, 1.43f, 0.608f, 0.0702f},
+                                        {7.73f, 0.649f, 0.291f, 7.4f, 0.925f, 0.00645f},
+                                        {7.29f, 1.0f, 0.697f, 10.6f, 1.44f, 0.149f},
+                                        {6.86f, 1.65f, 0.00716f, 7.06f, 1.96f, 0.174f}};
+    static_assert(prism::GM8_BK == prism::GW4_BK, "one K step for both");
+    const float* f = kBlocks[p.w8 ? 3 : p.w4 == 8 ? 2 : p.w4 / 4];
+    const uint32_t bm = p.w8 ? prism::GM8_BM : 32u * p.w4, bn = p.w8 ? prism::GM8_BN : prism::GW4_BN;
+    const uint64_t tiles = (uint64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn);
+    const float steps = (float)(K / prism::GW4_BK), fill = (float)tiles / (float)num_cu;
+    const float more = 0.25f * std::max(1.0f, fill) + 0.75f * rounds(tiles) - 1.0f;
+    return f[0] + steps * (f[1] + f[2] * std::min(1.0f, fill)) + more * (f[3] + steps * f[4]) + f[5] * mn;
   }
   const uint32_t rows = p.packed ? 32u * p.rt : 64u, blocks = (N + rows - 1) / rows;
   const uint32_t group = 32u * p.tt * (p.packed ? prism::kLkWaves / p.ks : 1u);
-  const uint64_t groups = (uint64_t)blocks * ((M + group - 1) / group) * p.split;
+  const float r = rounds((uint64_t)blocks * ((M + group - 1) / group) * p.split);
   const float steps = (float)((p.packed ? 2u : 1u) * ((p.per_split + p.ks - 1) / p.ks));
-  // MB of x that the row blocks read, and of partials that go out
+  // MB of x that the row blocks read; stores of single values, where N does not allow whole ones
   const float x_mb = (float)blocks * (float)M * (float)K * 2e-6f;
-  const float p_m = (float)p.split * (float)M * (float)N * 1e-6f;
+  const float odd = N % (p.packed && p.ks == 1 && p.split == 1 ? 8 : 4) ? (float)p.split * mn : 0.0f;
+  const float sum = p.split > 1 ? 1.0f : 0.0f, partials = sum * (float)p.split * mn;
+  const float astray = (uint64_t)K * bits / 8 % 16 ? r * steps : 0.0f;  // steps over index rows that are not aligned
+  const float unaligned = (uint64_t)M * N % 4 ? sum * (float)p.split : 0.0f;  // partials the sum reads one by one
   if (!p.packed) {
     // 32 and 64 tokens: fixed us (LUT loads, tables, sum, store), us per step; the same for each
-    // round after the first; us per MB of x; the sum's launch and its us per million partials
-    static const float kX[2][2][7] = {
-        {{4.15f, 0.64f, 2.2f, 0.74f, 0.03f, 1.9f, 1.7f}, {5.25f, 1.0f, 3.7f, 1.03f, 0.03f, 1.85f, 1.15f}},
-        {{4.55f, 0.545f, 2.95f, 0.68f, 0.05f, 2.2f, 1.55f}, {5.55f, 0.655f, 4.4f, 0.62f, 0.06f, 2.2f, 1.17f}}};
+    // round after the first; us per MB of x; the sum's launch and its us per million partials; us per
+    // million single stores, per split whose partials are not aligned, per step over unaligned rows
+    static const float kX[2][2][10] = {{{3.83f, 0.67f, 3.13f, 0.615f, 0.0379f, 2.26f, 0.522f, 1.06f, 0.494f, 0.215f},
+                                       {5.42f, 0.955f, 3.47f, 1.16f, 0.0248f, 1.99f, 2.0f, 0.792f, 0.441f, 0.619f}},
+                                      {{3.48f, 0.737f, 2.95f, 0.963f, 0.0364f, 2.87f, 0.67f, 0.0211f, 0.593f, 4.07e-06f},
+                                       {5.79f, 0.771f, 3.21f, 0.82f, 0.0485f, 2.34f, 1.79f, 0.714f, 0.502f, 0.2f}}};
     const float* f = kX[bits == 8][p.tt - 1];
-    return f[0] + steps * f[1] + (rounds(groups) - 1.0f) * (f[2] + steps * f[3]) + f[4] * x_mb +
-           (p.split > 1 ? f[5] + f[6] * p_m : 0.0f);
+    return f[0] + steps * f[1] + (r - 1.0f) * (f[2] + steps * f[3]) + f[4] * x_mb + f[5] * sum + f[6] * partials +
+           f[7] * odd + f[8] * unaligned + f[9] * astray;
   }
-  // 64 x 64 and 128 x 64 (4 bits) or 64 x 128 (8 bits) a wave: fixed us and us per step, more with
-  // all waves at work (not past M) and with each doubling of the waves on one token group, in whole
-  // rounds; us per MB of x; k_pack_x, a launch and its us per million elements; the sum as above
-  static const float kP[2][2][9] = {{{3.77f, 0.058f, 0.511f, 0.058f, 0.026f, 4.87f, 1.5f, 2.24f, 0.9f},
-                                     {7.78f, 0.108f, 0.62f, 0.058f, 0.059f, 4.42f, 1.34f, 1.87f, 0.87f}},
-                                    {{4.6f, 0.029f, 0.507f, 0.038f, 0.023f, 4.0f, 1.355f, 2.72f, 0.58f},
-                                     {8.86f, 0.113f, 0.616f, 0.033f, 0.02f, 4.08f, 1.31f, 2.39f, 0.64f}}};
+  // 64 x 64 and 128 x 64 (4 bits) or 64 x 128 (8 bits) a wave: per round fixed us and us per step, more
+  // with all waves at work (not past M) and with each doubling of the waves on one token group; us per
+  // MB of x; k_pack_x, a launch and its us per million elements; the sum and the stores as above
+  static const float kP[2][2][12] = {
+      {{4.65f, 0.0707f, 0.535f, 0.0525f, 0.0217f, 3.81f, 1.59f, 3.83f, 0.461f, 2.29f, 0.227f, 0.101f},
+       {8.92f, 0.247f, 0.562f, 0.0599f, 0.0468f, 3.88f, 0.974f, 4.65f, 0.782f, 1.76f, 1.05f, 0.213f}},
+      {{4.23f, 0.0878f, 0.523f, 0.0835f, 0.0128f, 3.54f, 1.01f, 4.22f, 0.709f, 2.44f, 0.283f, 0.0148f},
+       {9.29f, 0.122f, 0.709f, 0.0508f, 0.0137f, 3.22f, 0.575f, 3.1f, 1.07f, 2.4f, 0.774f, 0.062f}}};
   const float* f = kP[bits == 8][p.rt * p.tt > 4];
   const float live = std::min(1.0f, (float)(p.ks * ((M + 32u * p.tt - 1) / (32u * p.tt))) / (float)prism::kLkWaves);
   const float doublings = p.ks == 8 ? 3.0f : p.ks == 4 ? 2.0f : p.ks == 2 ? 1.0f : 0.0f;
-  return (float)((groups + num_cu - 1) / num_cu) * (f[0] + steps * (f[1] + (f[2] + doublings * f[3]) * live)) +
-         f[4] * x_mb + f[5] + f[6] * (float)M * (float)K * 1e-6f + (p.split > 1 ? f[7] + f[8] * p_m : 0.0f);
+  return r * (f[0] + steps * (f[1] + (f[2] + doublings * f[3]) * live)) + f[4] * x_mb + f[5] +
+         f[6] * (float)M * (float)K * 1e-6f + f[7] * sum + f[8] * partials + f[9] * odd +
+         f[10] * unaligned + f[11] * astray;
 }
 
 // Where a call's scratch (packed X, partials) comes from: kept memory, the pool
 // for this call, or none may be used.
 enum class Scratch { kKept, kCall, kNone };
 
-// The fastest plan by that estimate.
-//  * k_gemm_lookup_x, to 256 tokens where there is another (X unpacked costs no
-//    launch, but is read again by each 64 rows: 14336 x 4096, 33 tokens 13.6 us
-//    against 20.5 packed, 128 tokens 29.5 against 22.8);
-//  * k_gemm_lookup above 64;
-//  * k_gemm_w4, which decodes each block's weights once, above 32: from half a
-//    block for each CU on (151936 x 896 at 64 / 128 / 256 tokens 34.7 / 58.8 /
-//    92.8 us against 65.3 / 85.7 / 112), and above 256 wherever the estimate
-//    says so (18944 x 3584, 768 tokens 98 against 113 us, 14336 x 4096, 1024
-//    tokens 113 against 115).
-//  * k_gemm8 where no scratch may be used, above 256 tokens at 8 bits (14336 x
-//    4096, 2048 tokens 441 us against 577 in k_gemm_lookup_x, 300 tokens 112
-//    against 85).
-// Of plans that the estimate cannot tell apart, the one in a single launch goes
-// first, then the lookup GEMM (4 and 7 %: 4096 x 14336, 203 tokens, 44.9 us
-// unpacked against 46.3; 14336 x 4096, 2048 tokens, 219 packed against 225).
+// The fastest plan by that estimate.  Every kernel is ahead somewhere (MI355X,
+// with scratch kept, us of the fastest plan of each):
+//  * k_gemm_lookup_x, up to 32 tokens the only one: above them in blocks of 32 tokens
+//    where those fill the CUs better (2752 x 1792, 128 tokens 7.0 against 9.8 in
+//    blocks of 64), and of 64 where 32 take more rounds (14336 x 4096, 33 tokens
+//    14.5);
+//  * k_gemm_lookup above 32 tokens: X is packed once and not read unpacked by each 64
+//    rows (14336 x 4096, 256 tokens 39 against 52);
+//  * k_gemm_w4, which decodes each block's weights once, above 32 (151936 x 896,
+//    64 tokens 34.7 against 65.3); with 3 % for the others, as its times move most
+//    from card to card (14336 x 4096, 2048 tokens 221..236);
+//  * k_gemm8 where no scratch may be used, above 256 tokens at 8 bits (14336 x 4096,
+//    2048 tokens 441 against 577 in k_gemm_lookup_x).
 // Scratch of the call's own is allocated and freed on each call: 3..5 us more, and
 // no call below about 22 us of host time (14336 x 4096, 80 / 300 tokens 23.6 / 51.5
 // us with kept scratch, 28.6 / 54.4 with its own).
@@ -1364,7 +1368,12 @@ GemmPlan plan_gemm(uint32_t bits, uint32_t M, uint32_t N, uint32_t K, uint32_t n
   // (weights that run_gemm cuts into row slabs have no partials)
   const uint32_t max_split = (uint64_t)N * K * bits / 8 < kMaxIndexBytes ? 16 : 1;
   auto consider = [&](bool packed, int rt, int tt, uint32_t ks) {
-    for (uint32_t split = 1; split <= max_split; split *= 2) {
+    // (not with half the waves past M, nor splits of what fills the CUs four times: 1..2 us of host
+    // time at 33..64 tokens)
+    const uint32_t tiles = (M + 32u * tt - 1) / (32u * tt), waves = packed ? prism::kLkWaves / ks : 1;
+    if (waves >= 2 * tiles) return;
+    const uint64_t groups = (uint64_t)(N / (32u * rt)) * ((tiles + waves - 1) / waves);
+    for (uint32_t split = 1; split <= max_split && (split == 1 || groups * split < 8 * num_cu); split *= 2) {
       GemmPlan p;
       p.packed = packed;
       p.rt = rt;
@@ -1374,16 +1383,13 @@ GemmPlan plan_gemm(uint32_t bits, uint32_t M, uint32_t N, uint32_t K, uint32_t n
       if (!plan_sizes(&p, bits, M, N, K)) continue;
       if (scratch == Scratch::kNone && p.x_bytes + p.p_bytes) continue;
       p.us = gemm_plan_us(p, bits, M, N, K, num_cu);
-      if (p.x_bytes + p.p_bytes) p.us *= 1.04f;
       if (scratch == Scratch::kCall && p.x_bytes + p.p_bytes) p.us = std::max(p.us + 4.0f, 22.0f);
       if (p.us < best.us) best = p;
     }
   };
-  if (M <= 256 || scratch == Scratch::kNone) {
-    if (M <= 64) consider(false, 2, 1, prism::kLkWaves);
-    if (M > 32) consider(false, 2, 2, prism::kLkWaves);
-  }
-  if (M > 64)
+  consider(false, 2, 1, prism::kLkWaves);
+  if (M > 32) {
+    consider(false, 2, 2, prism::kLkWaves);
     for (uint32_t ks = 1; ks <= prism::kLkWaves; ks *= 2) {
       consider(true, 2, 2, ks);
       if (bits == 4)
@@ -1391,14 +1397,13 @@ GemmPlan plan_gemm(uint32_t bits, uint32_t M, uint32_t N, uint32_t K, uint32_t n
       else
         consider(true, 2, 4, ks);
     }
+  }
   if (bits == 4 && M > 32 && K % prism::GW4_BK == 0 && (uint64_t)N * (K / 2) < (1ull << 31) &&
       (uint64_t)K * 512 < (1ull << 31))
     for (int mi = 2; mi <= 8; mi *= 2) {
-      const uint64_t tiles = (uint64_t)((M + 32u * mi - 1) / (32u * mi)) * ((N + prism::GW4_BN - 1) / prism::GW4_BN);
-      if (M <= 256 && 2 * tiles < num_cu) continue;
       GemmPlan p;
       p.w4 = mi;
-      p.us = 1.07f * gemm_plan_us(p, bits, M, N, K, num_cu);
+      p.us = 1.03f * gemm_plan_us(p, bits, M, N, K, num_cu);
       if (p.us < best.us) best = p;
     }
   if (bits == 8 && scratch == Scratch::kNone && M > 256 && K % prism::GM8_BK == 0) {
@@ -1416,29 +1421,37 @@ GemmPlan plan_gemm(uint32_t bits, uint32_t M, uint32_t N, uint32_t K, uint32_t n
 }
 
 // Estimated time of M vectors (5..32; over GI weights 9 and more) as GEMV passes, us on MI355X:
-// the matrix-core GEMV in passes of 16 where it runs, fixed us, then for each
-// round of workgroups a fixed part and us per 1000 elements of K, with none and
-// with each vector; else the tile GEMV in passes of 8 vectors (fewer for long
-// rows), fixed us, more for each doubling of its vectors, and us per million
-// weights, with none and with each vector; no pass below the weights' bytes at 5.5
-// TB/s.  Fitted to the passes of the same 22 shapes, within 6..15 % (root mean
-// square).
+//  * the matrix-core GEMV in passes of 16 where it runs: fixed us, then for each round
+//    of workgroups a fixed part and us per 1000 elements of K, with none and with each
+//    vector; and us per 1000 elements of K and row that the last workgroup lacks, whose
+//    lanes all look up the last row's elements in one LDS bank;
+//  * else over GI weights lane-per-row passes of two;
+//  * else the tile GEMV in passes of 8 vectors (fewer for long rows): fixed us, more
+//    for each doubling of its vectors, us per million weights, with none and with each
+//    vector, and with each vector us per million rows and per 1000 elements of K.
+// No pass is below a multiple of the weights' bytes at 5.5 TB/s.  Fitted to the
+// passes of 450 shapes, within 4 (4 bits) and 8..10 % (8 bits, tile) root mean square.
 float passes_us(uint32_t bits, uint32_t gi, uint32_t M, uint32_t N, uint32_t K, uint32_t num_cu) {
   const bool near = (uint64_t)N * K * bits / 8 < (1ull << 31);
   const float floor_us = (float)N * ((float)K * (float)bits / 8 + (float)(2u << bits)) / 5.5e6f;  // the weights' bytes
+  const float k = (float)K * 1e-3f, m = (float)N * 1e-6f;
   float us = 0.0f;
+  if (gi && bits == 4 && K % prism::kGmGroup != 0) return (float)((M + 1) / 2) * 1.4f * floor_us;
   if (gi || (K % prism::kGmGroup == 0 && N >= 4096 && near)) {
-    static const float kMfma[2][2][4] = {{{0.43f, 2.5f, 0.66f, 0.048f}, {0.3f, 3.6f, 1.35f, 0.05f}},
-                                         {{7.0f, 1.2f, 0.0f, 0.07f}, {0.0f, 17.0f, 0.0f, 0.08f}}};
-    const float* f = kMfma[gi != 0][bits == 8];
-    const float rounds = (float)(((N + 63) / 64 + num_cu - 1) / num_cu);
+    static const float kMfma[2][2][6] = {
+        {{2.59f, 0.66f, 0.82f, 0.033f, 1.2f, 0.012f}, {3.3f, 0.15f, 0.487f, 0.04f, 1.25f, 0.012f}},
+        {{3.02f, 1.26f, 1.365f, 0.048f, 1.23f, 0.13f}, {4.69f, 0.0f, 1.09f, 0.043f, 1.31f, 0.13f}}};
+    const float* f = kMfma[bits == 8][gi != 0];
+    const float rounds = (float)(((N + prism::kGmRows - 1) / prism::kGmRows + num_cu - 1) / num_cu);
+    const float lacks = k * (float)((prism::kGmRows - N % prism::kGmRows) % prism::kGmRows);
     for (uint32_t n = M; n; n -= std::min(n, 16u))
-      us += std::max(floor_us, f[0] + rounds * (f[1] + (float)K * 1e-3f * (f[2] + f[3] * (float)std::min(n, 16u))));
+      us += std::max(f[4] * floor_us,
+                     f[0] + rounds * (f[1] + k * (f[2] + f[3] * (float)std::min(n, 16u))) + f[5] * lacks);
     return us;
   }
-  static const float kTile[2][4] = {{2.8f, 0.47f, 0.078f, 0.032f}, {3.4f, 0.23f, 0.161f, 0.039f}};
+  static const float kTile[2][7] = {{2.77f, 0.377f, 0.027f, 0.039f, 16.4f, 0.027f, 2.18f},
+                                    {2.84f, 0.2f, 0.184f, 0.012f, 75.0f, 0.049f, 1.55f}};
   const float* f = kTile[bits == 8];
-  const float mw = (float)N * (float)K * 1e-6f;
   for (uint32_t n = M; n;) {
     uint32_t c = std::min(n, 8u), nb, lg;
     for (;; c = nb / 2) {  // vectors of a pass whose x fits the registers of 8 waves
@@ -1446,7 +1459,8 @@ float passes_us(uint32_t bits, uint32_t gi, uint32_t M, uint32_t N, uint32_t K, 
       if (near && (K / 8 + 511) / 512 <= std::min(8u, 16 / nb)) break;
       if (nb == 1) return 3.4e38f;  // the generic kernel, whatever it takes
     }
-    us += std::max(floor_us, f[0] + f[1] * (float)lg + mw * (f[2] + f[3] * (float)nb));
+    us += std::max(f[6] * floor_us, f[0] + f[1] * (float)lg + m * (float)K * (f[2] + f[3] * (float)nb) +
+                                        (float)nb * (f[4] * m + f[5] * k));
     n -= c;
   }
   return us;
@@ -1465,18 +1479,15 @@ bool gemm_can(const prism_hip_weight* w, const void* d_x, uint32_t M, bool gemv)
 }
 
 // Whether the plan goes ahead of passes: above 32 tokens always, else by both
-// estimates, with 5 % for passes.  MI355X, plan against passes on the context's
-// stream: 14336 x 4096, 32 tokens, 4 bits 9.4 against 23.0 us, 16 tokens 9.2 against
-// 12.1; 4096 x 14336, 8 tokens 12.0 against 18.5, but 19.9 where it cannot split K
+// estimates, with 3 % for passes (0.5 % over the faster side on average, at most 27).  MI355X, plan
+// against passes on the context's stream: 14336 x 4096, 32 tokens, 4 bits 9.4
+// against 23.0 us, 16 tokens 9.2 against 12.1; 14592 x 13184, 14 tokens 20.5 against
+// 31.1; 4096 x 14336, 8 tokens 12.0 against 18.5, but 19.9 where it cannot split K
 // (a caller's stream, capture: 24.3); 4096 x 4096, 9 tokens 8.4 against 6.9; 256 x
-// 8192, 8 tokens 8.5 against 6.0, captured 15.8 against 7.1.  Up to 16 tokens the
-// matrix-core GEMV keeps what takes the lookup GEMM more than one round (18944 x
-// 3584, 12 tokens 13.7 against 16.0).
+// 8192, 8 tokens 8.5 against 6.0, captured 15.8 against 7.1; 151936 x 896, 8
+// tokens, 8 bits 76 against 57.
 bool gemm_goes_first(const prism_hip_ctx* ctx, const prism_hip_weight* w, uint32_t M, const GemmPlan& p) {
-  if (M > 32) return true;
-  const uint32_t N = w->dim_m, K = w->dim_n, num_cu = (uint32_t)ctx->num_cu;
-  if (M <= 16 && K % prism::kGmGroup == 0 && (N + 63) / 64 > num_cu) return false;
-  return 1.05f * p.us < passes_us(w->bits, w->gi, M, N, K, num_cu);
+  return M > 32 || 1.03f * p.us < passes_us(w->bits, w->gi, M, w->dim_m, w->dim_n, (uint32_t)ctx->num_cu);
 }
 
 // A call on the context's stream uses its buffer, one on a caller's stream memory
