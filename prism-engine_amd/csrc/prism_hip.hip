@@ -1280,23 +1280,24 @@ int run_gemm(prism_hip_ctx* ctx, const prism_hip_weight* w, GemmPlan p, const vo
   return PRISM_HIP_OK;
 }
 
-// Estimated time of a plan in us on MI355X.  Fitted to every plan of 580 shapes
-// (64 .. 151936 rows of 768 .. 16384, odd ones among them) at 5 to 11 numbers of
-// tokens each from 5 to 2048, for the least time lost by the plan it picks: with
-// scratch 0.5 % over the fastest plan on average, one in twenty over 4 %, at most 19;
-// without, 0.1 % and at most 24.  (Shapes left out of the fit: 0.6 and 0.1 %, at most
-// 17 and 14.)
-float gemm_plan_us(const GemmPlan& p, uint32_t bits, uint32_t M, uint32_t N, uint32_t K, uint32_t num_cu) {
+// Estimated time of a plan in us on MI355X.  Fitted to every plan of 730 shapes
+// (64 .. 151936 rows of 768 .. 16384, odd ones among them) at 5 to 17 numbers of
+// tokens each from 5 to 2048, over weights in the Infinity Cache and over as many
+// that they are not, for the least time lost by the plan it picks: with scratch 0.5 %
+// over the fastest plan on average, one in twenty over 4 %, at most 26; without, 0.1 %
+// and at most 20.  (Shapes left out of the fit: 0.7 and 0.1 %, at most 19 and 14.)
+float gemm_plan_us(const GemmPlan& p, uint32_t bits, uint32_t gi, uint32_t M, uint32_t N, uint32_t K,
+                   uint32_t num_cu) {
   const float mn = (float)M * (float)N * 1e-6f;
   auto rounds = [&](uint64_t groups) { return (float)((groups + num_cu - 1) / num_cu); };  // over the CUs
   if (p.w4 || p.w8) {
     // k_gemm_w4 of 64, 128 and 256 tokens, k_gemm8: fixed us, us per step, more with all CUs busy; the
     // same for each round after the first, of which a last one that is not full counts a quarter for
     // its share of the CUs; us per million outputs
-    static const float kBlocks[4][6] = {{4.63f, 0.681f, 0.0327f, 1.43f, 0.608f, 0.0702f},
-                                        {7.73f, 0.649f, 0.291f, 7.4f, 0.925f, 0.00645f},
-                                        {7.29f, 1.0f, 0.697f, 10.6f, 1.44f, 0.149f},
-                                        {6.86f, 1.65f, 0.00716f, 7.06f, 1.96f, 0.174f}};
+    static const float kBlocks[4][6] = {{4.09f, 0.728f, 0.0129f, 2.68f, 0.594f, 0.0484f},
+                                        {8.49f, 0.685f, 0.212f, 10.6f, 0.846f, 0.0242f},
+                                        {12.8f, 1.1f, 0.344f, 13.6f, 1.5f, 0.0559f},
+                                        {10.1f, 1.54f, 0.0145f, 12.6f, 1.67f, 0.0112f}};
     static_assert(prism::GM8_BK == prism::GW4_BK, "one K step for both");
     const float* f = kBlocks[p.w8 ? 3 : p.w4 == 8 ? 2 : p.w4 / 4];
     const uint32_t bm = p.w8 ? prism::GM8_BM : 32u * p.w4, bn = p.w8 ? prism::GM8_BN : prism::GW4_BN;
@@ -1314,33 +1315,37 @@ float gemm_plan_us(const GemmPlan& p, uint32_t bits, uint32_t M, uint32_t N, uin
   const float odd = N % (p.packed && p.ks == 1 && p.split == 1 ? 8 : 4) ? (float)p.split * mn : 0.0f;
   const float sum = p.split > 1 ? 1.0f : 0.0f, partials = sum * (float)p.split * mn;
   const float astray = (uint64_t)K * bits / 8 % 16 ? r * steps : 0.0f;  // steps over index rows that are not aligned
+  const float apart = gi ? 0.0f : r * steps;  // steps whose lanes read index rows apart, not GI groups
   const float unaligned = (uint64_t)M * N % 4 ? sum * (float)p.split : 0.0f;  // partials the sum reads one by one
   if (!p.packed) {
     // 32 and 64 tokens: fixed us (LUT loads, tables, sum, store), us per step; the same for each
     // round after the first; us per MB of x; the sum's launch and its us per million partials; us per
     // million single stores, per split whose partials are not aligned, per step over unaligned rows
-    static const float kX[2][2][10] = {{{3.83f, 0.67f, 3.13f, 0.615f, 0.0379f, 2.26f, 0.522f, 1.06f, 0.494f, 0.215f},
-                                       {5.42f, 0.955f, 3.47f, 1.16f, 0.0248f, 1.99f, 2.0f, 0.792f, 0.441f, 0.619f}},
-                                      {{3.48f, 0.737f, 2.95f, 0.963f, 0.0364f, 2.87f, 0.67f, 0.0211f, 0.593f, 4.07e-06f},
-                                       {5.79f, 0.771f, 3.21f, 0.82f, 0.0485f, 2.34f, 1.79f, 0.714f, 0.502f, 0.2f}}};
+    // and over rows that are not GI
+    static const float kX[2][2][11] = {
+        {{3.81f, 0.57f, 2.5f, 0.752f, 0.0172f, 2.12f, 1.35f, 0.202f, 0.568f, 0.0894f, 0.296f},
+         {5.59f, 0.914f, 3.1f, 1.23f, 0.0213f, 2.16f, 2.29f, 0.189f, 0.438f, 0.469f, 0.13f}},
+        {{3.56f, 0.509f, 3.81f, 0.461f, 0.033f, 2.83f, 0.127f, 0.0018f, 0.626f, 0.0f, 0.364f},
+         {6.07f, 0.747f, 3.52f, 0.664f, 0.0284f, 2.16f, 1.76f, 1.01f, 0.444f, 0.148f, 0.19f}}};
     const float* f = kX[bits == 8][p.tt - 1];
     return f[0] + steps * f[1] + (r - 1.0f) * (f[2] + steps * f[3]) + f[4] * x_mb + f[5] * sum + f[6] * partials +
-           f[7] * odd + f[8] * unaligned + f[9] * astray;
+           f[7] * odd + f[8] * unaligned + f[9] * astray +
+           f[10] * apart;
   }
   // 64 x 64 and 128 x 64 (4 bits) or 64 x 128 (8 bits) a wave: per round fixed us and us per step, more
   // with all waves at work (not past M) and with each doubling of the waves on one token group; us per
   // MB of x; k_pack_x, a launch and its us per million elements; the sum and the stores as above
-  static const float kP[2][2][12] = {
-      {{4.65f, 0.0707f, 0.535f, 0.0525f, 0.0217f, 3.81f, 1.59f, 3.83f, 0.461f, 2.29f, 0.227f, 0.101f},
-       {8.92f, 0.247f, 0.562f, 0.0599f, 0.0468f, 3.88f, 0.974f, 4.65f, 0.782f, 1.76f, 1.05f, 0.213f}},
-      {{4.23f, 0.0878f, 0.523f, 0.0835f, 0.0128f, 3.54f, 1.01f, 4.22f, 0.709f, 2.44f, 0.283f, 0.0148f},
-       {9.29f, 0.122f, 0.709f, 0.0508f, 0.0137f, 3.22f, 0.575f, 3.1f, 1.07f, 2.4f, 0.774f, 0.062f}}};
+  static const float kP[2][2][13] = {
+      {{3.85f, 0.0931f, 0.517f, 0.0701f, 0.0234f, 4.0f, 1.25f, 4.04f, 0.52f, 2.01f, 0.171f, 0.0151f, 0.104f},
+       {7.7f, 0.246f, 0.546f, 0.0936f, 0.0383f, 4.56f, 0.444f, 5.18f, 0.904f, 2.26f, 0.365f, 0.00727f, 0.317f}},
+      {{4.15f, 0.0812f, 0.498f, 0.121f, 0.0111f, 3.54f, 0.912f, 4.91f, 0.837f, 2.56f, 0.252f, 0.0263f, 0.0236f},
+       {9.37f, 0.0948f, 0.769f, 0.0749f, 0.00277f, 4.15f, 0.435f, 3.04f, 1.45f, 2.44f, 0.651f, 0.0953f, 0.000496f}}};
   const float* f = kP[bits == 8][p.rt * p.tt > 4];
   const float live = std::min(1.0f, (float)(p.ks * ((M + 32u * p.tt - 1) / (32u * p.tt))) / (float)prism::kLkWaves);
   const float doublings = p.ks == 8 ? 3.0f : p.ks == 4 ? 2.0f : p.ks == 2 ? 1.0f : 0.0f;
   return r * (f[0] + steps * (f[1] + (f[2] + doublings * f[3]) * live)) + f[4] * x_mb + f[5] +
          f[6] * (float)M * (float)K * 1e-6f + f[7] * sum + f[8] * partials + f[9] * odd +
-         f[10] * unaligned + f[11] * astray;
+         f[10] * unaligned + f[11] * astray + f[12] * apart;
 }
 
 // Where a call's scratch (packed X, partials) comes from: kept memory, the pool
@@ -1356,14 +1361,14 @@ enum class Scratch { kKept, kCall, kNone };
 //  * k_gemm_lookup above 32 tokens: X is packed once and not read unpacked by each 64
 //    rows (14336 x 4096, 256 tokens 39 against 52);
 //  * k_gemm_w4, which decodes each block's weights once, above 32 (151936 x 896,
-//    64 tokens 34.7 against 65.3); with 3 % for the others, as its times move most
-//    from card to card (14336 x 4096, 2048 tokens 221..236);
+//    64 tokens 34.7 against 65.3);
 //  * k_gemm8 where no scratch may be used, above 256 tokens at 8 bits (14336 x 4096,
 //    2048 tokens 441 against 577 in k_gemm_lookup_x).
 // Scratch of the call's own is allocated and freed on each call: 3..5 us more, and
 // no call below about 22 us of host time (14336 x 4096, 80 / 300 tokens 23.6 / 51.5
 // us with kept scratch, 28.6 / 54.4 with its own).
-GemmPlan plan_gemm(uint32_t bits, uint32_t M, uint32_t N, uint32_t K, uint32_t num_cu, Scratch scratch) {
+GemmPlan plan_gemm(uint32_t bits, uint32_t gi, uint32_t M, uint32_t N, uint32_t K, uint32_t num_cu,
+                   Scratch scratch) {
   GemmPlan best;
   // (weights that run_gemm cuts into row slabs have no partials)
   const uint32_t max_split = (uint64_t)N * K * bits / 8 < kMaxIndexBytes ? 16 : 1;
@@ -1382,7 +1387,7 @@ GemmPlan plan_gemm(uint32_t bits, uint32_t M, uint32_t N, uint32_t K, uint32_t n
       p.split = split;
       if (!plan_sizes(&p, bits, M, N, K)) continue;
       if (scratch == Scratch::kNone && p.x_bytes + p.p_bytes) continue;
-      p.us = gemm_plan_us(p, bits, M, N, K, num_cu);
+      p.us = gemm_plan_us(p, bits, gi, M, N, K, num_cu);
       if (scratch == Scratch::kCall && p.x_bytes + p.p_bytes) p.us = std::max(p.us + 4.0f, 22.0f);
       if (p.us < best.us) best = p;
     }
@@ -1403,13 +1408,13 @@ GemmPlan plan_gemm(uint32_t bits, uint32_t M, uint32_t N, uint32_t K, uint32_t n
     for (int mi = 2; mi <= 8; mi *= 2) {
       GemmPlan p;
       p.w4 = mi;
-      p.us = 1.03f * gemm_plan_us(p, bits, M, N, K, num_cu);
+      p.us = gemm_plan_us(p, bits, gi, M, N, K, num_cu);
       if (p.us < best.us) best = p;
     }
   if (bits == 8 && scratch == Scratch::kNone && M > 256 && K % prism::GM8_BK == 0) {
     GemmPlan p;
     p.w8 = true;
-    p.us = gemm_plan_us(p, bits, M, N, K, num_cu);
+    p.us = gemm_plan_us(p, bits, gi, M, N, K, num_cu);
     if (p.us < best.us) best = p;
   }
   if (best.us > 3e38f) {  // rows too long for the scratch: the kernel that needs none
@@ -1439,8 +1444,8 @@ float passes_us(uint32_t bits, uint32_t gi, uint32_t M, uint32_t N, uint32_t K, 
   if (gi && bits == 4 && K % prism::kGmGroup != 0) return (float)((M + 1) / 2) * 1.4f * floor_us;
   if (gi || (K % prism::kGmGroup == 0 && N >= 4096 && near)) {
     static const float kMfma[2][2][6] = {
-        {{2.59f, 0.66f, 0.82f, 0.033f, 1.2f, 0.012f}, {3.3f, 0.15f, 0.487f, 0.04f, 1.25f, 0.012f}},
-        {{3.02f, 1.26f, 1.365f, 0.048f, 1.23f, 0.13f}, {4.69f, 0.0f, 1.09f, 0.043f, 1.31f, 0.13f}}};
+        {{2.59f, 0.67f, 0.83f, 0.031f, 1.2f, 0.004f}, {3.3f, 0.17f, 0.465f, 0.042f, 1.32f, 0.007f}},
+        {{3.0f, 1.27f, 1.36f, 0.048f, 1.22f, 0.13f}, {4.67f, 0.0f, 1.06f, 0.045f, 1.29f, 0.13f}}};
     const float* f = kMfma[bits == 8][gi != 0];
     const float rounds = (float)(((N + prism::kGmRows - 1) / prism::kGmRows + num_cu - 1) / num_cu);
     const float lacks = k * (float)((prism::kGmRows - N % prism::kGmRows) % prism::kGmRows);
@@ -1449,8 +1454,8 @@ float passes_us(uint32_t bits, uint32_t gi, uint32_t M, uint32_t N, uint32_t K, 
                      f[0] + rounds * (f[1] + k * (f[2] + f[3] * (float)std::min(n, 16u))) + f[5] * lacks);
     return us;
   }
-  static const float kTile[2][7] = {{2.77f, 0.377f, 0.027f, 0.039f, 16.4f, 0.027f, 2.18f},
-                                    {2.84f, 0.2f, 0.184f, 0.012f, 75.0f, 0.049f, 1.55f}};
+  static const float kTile[2][7] = {{2.8f, 0.343f, 0.025f, 0.039f, 20.5f, 0.026f, 2.2f},
+                                    {2.78f, 0.22f, 0.178f, 0.014f, 75.0f, 0.048f, 1.56f}};
   const float* f = kTile[bits == 8];
   for (uint32_t n = M; n;) {
     uint32_t c = std::min(n, 8u), nb, lg;
@@ -1479,7 +1484,7 @@ bool gemm_can(const prism_hip_weight* w, const void* d_x, uint32_t M, bool gemv)
 }
 
 // Whether the plan goes ahead of passes: above 32 tokens always, else by both
-// estimates, with 3 % for passes (0.5 % over the faster side on average, at most 27).  MI355X, plan
+// estimates, with 3 % for passes (0.4 % over the faster side on average, at most 27).  MI355X, plan
 // against passes on the context's stream: 14336 x 4096, 32 tokens, 4 bits 9.4
 // against 23.0 us, 16 tokens 9.2 against 12.1; 14592 x 13184, 14 tokens 20.5 against
 // 31.1; 4096 x 14336, 8 tokens 12.0 against 18.5, but 19.9 where it cannot split K
@@ -1508,7 +1513,7 @@ int launch_gemm(prism_hip_ctx* ctx, const prism_hip_weight* w, const void* d_X, 
     Scratch sc = Scratch::kKept;  // (`fixed` is)
     const int rc = fixed ? PRISM_HIP_OK : scratch_of(ctx, st, &sc);
     if (rc) return rc;
-    const GemmPlan p = plan_gemm(w->bits, M, w->dim_m, w->dim_n, (uint32_t)ctx->num_cu, sc);
+    const GemmPlan p = plan_gemm(w->bits, w->gi, M, w->dim_m, w->dim_n, (uint32_t)ctx->num_cu, sc);
     if (gemm_goes_first(ctx, w, M, p)) return run_gemm(ctx, w, p, d_X, M, d_Y, st, fixed);
   }
   return launch_gemv_passes(ctx, w, nullptr, d_X, M, d_Y, st);

@@ -25,15 +25,15 @@ CASES = [
     (4, 129, 136, 257, "x"), (4, 257, 1000, 300, "x"), (4, 1001, 1032, 513, "x"), (4, 3, 8, 270, "x"),
     (4, 640, 648, 511, "x"), (4, 9100, 2112, 230, "p"), (4, 3584, 2048, 300, "p"),
     # k_gemm_w4 of 2, 4 and 8 token tiles, one K step and more, GI groups of 40
-    (4, 40000, 64, 64, "w"), (4, 33000, 128, 33, "w"), (4, 32900, 192, 129, "w"), (4, 32900, 192, 255, "w"),
+    (4, 40000, 64, 64, "w"), (4, 33000, 128, 33, "w"), (4, 32900, 192, 129, "w"), (4, 32900, 192, 255, "w"), (4, 32900, 512, 255, "w"), (4, 20700, 192, 600, "w"),
     (4, 16500, 512, 300, "w"), (4, 9100, 2112, 400, "w"),
     (8, 64, 32, 17, "x"), (8, 66, 40, 10, "x"), (8, 130, 1000, 33, "x"), (8, 200, 2048, 64, "x"), (8, 9100, 2048, 20, "x"),
-    (8, 129, 64, 257, "x"), (8, 255, 72, 290, "x"), (8, 1001, 1032, 300, "x"), (8, 9100, 2048, 290, "p"),
+    (8, 129, 64, 257, "x"), (8, 255, 72, 290, "x"), (8, 1001, 1032, 300, "x"), (8, 9100, 2048, 200, "p"),
     (8, 5, 8, 266, "x"),
     # packed X over row tiles of 64 and 128 and token tiles of 64 and 128, one iteration of K and more, K split
     (4, 3329, 88, 403, "p"), (4, 12547, 176, 137, "p"), (4, 5309, 896, 198, "p"), (4, 3328, 4760, 282, "p"),
     (4, 8269, 304, 566, "p"), (4, 9321, 2968, 142, "p"), (8, 4235, 64, 791, "p"), (8, 7816, 128, 261, "p"),
-    (8, 4678, 144, 441, "p"), (8, 8575, 360, 112, "p"), (8, 5761, 2432, 141, "p"), (8, 972, 2240, 1068, "p"),
+    (8, 4678, 144, 441, "p"), (8, 8575, 360, 112, "p"), (8, 5761, 2432, 200, "p"), (8, 972, 2240, 1068, "p"),
     (8, 15645, 208, 627, "p"), (8, 9751, 296, 723, "p"),
 ]
 
