@@ -568,7 +568,7 @@ def run_palettize(args, pe, seed) -> int:
                    "k": 16, "max_iter": 50, "seed": seed},
         "roofline": {"bound": "hbm", "achieved": round(gbs, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(gbs / HBM_PEAK_GBS, 5), "traffic": None,
-                     "kernel": "k_palettize (whole model: fp32 read + payload write per step)",
+                     "kernel": "k_palettize_rows (whole model: fp32 read + payload write per step)",
                      "algorithmic_per_launch": params * 4 + out_bytes},
         "cpu_baseline": cpu,
     }

@@ -232,9 +232,10 @@ __global__ __launch_bounds__(256) void k_pack_x(const uint16_t* __restrict__ X, 
 //    to the compiler the loads sank to their uses or the loop spilled.
 //  * KS > 1: the slices' tiles are added pairwise in a fixed tree, each wave
 //    handing its partner half of what it holds.
-// Bounded by the matrix cores and, at 8 bits, the LDS: 14336 x 4096 x 512 at
-// 4 bits, KS = 1: a wave's loop takes 75..84 us where its SIMD's MFMAs alone
-// take 62.  The lookups' LDS time is 16 % of the kernel (no bank conflicts).
+// Bounded by no single unit: at 14336 x 4096 x 2048 the matrix cores are busy for 63 %
+// (4 bits) and 50 % (8 bits) of the cycles, the lookups' LDS for 33 and 27 (no bank
+// conflicts), the VALU for 30, and a wave waits for 36..40 % of its time; the clock falls
+// to 1.7 GHz.
 template <int BITS, int RT, int TT, bool RAGGED>
 __global__ __launch_bounds__(512) void k_gemm_lookup(LkArgs a) {
   using S = LkShape<BITS>;
