@@ -1150,8 +1150,8 @@ hipError_t ensure_gemm_scratch(prism_hip_ctx* ctx, size_t bytes) {
 }
 
 // The plan's scratch sizes and the tokens one launch takes (all of M, or with
-// a large M as many as keep packed X within the scratch); false when the
-// partials do not fit.
+// a large M as many as keep packed X within the scratch and the launch below 2^32
+// threads); false when the partials do not fit.
 bool plan_sizes(GemmPlan* p, uint32_t bits, uint32_t M, uint32_t N, uint32_t K) {
   const uint32_t step = prism::lk_step(bits);
   const uint32_t units = p->packed ? (K + 2 * step - 1) / (2 * step) : (K + step - 1) / step;
@@ -1159,17 +1159,18 @@ bool plan_sizes(GemmPlan* p, uint32_t bits, uint32_t M, uint32_t N, uint32_t K) 
   p->split = (units + p->per_split - 1) / p->per_split;
   p->tokens = M;
   p->x_bytes = p->p_bytes = 0;
-  if (p->packed) {
-    const size_t tile = (size_t)units * 2 * step * 64;  // 32 tokens
-    const uint32_t group = (uint32_t)p->tt * (prism::kLkWaves / p->ks);
-    size_t fit = kGemmScratchBytes / tile;
-    if (fit < (M + 31) / 32) {
-      if (fit > group) fit = fit / group * group;
-      if (fit == 0 || p->split > 1) return false;
-      p->tokens = (uint32_t)fit * 32;
-    }
-    p->x_bytes = (p->tokens + 31) / 32 * tile;
+  // in tiles of 32 tokens: a workgroup's, what launch and scratch hold
+  const uint32_t rows = p->packed ? 32u * p->rt : 64u;
+  const uint32_t group = (uint32_t)p->tt * (p->packed ? prism::kLkWaves / p->ks : 1);
+  const size_t tile = p->packed ? (size_t)units * 2 * step * 64 : 0;
+  size_t fit = std::max<size_t>(1, 0xFFFFFFFFu / (64 * prism::kLkWaves) / ((N + rows - 1) / rows)) * group;
+  if (p->packed) fit = std::min(fit, kGemmScratchBytes / tile);
+  if (fit < (M + 31) / 32) {
+    if (fit > group) fit = fit / group * group;
+    if (fit == 0 || p->split > 1) return false;
+    p->tokens = (uint32_t)fit * 32;
   }
+  if (p->packed) p->x_bytes = (p->tokens + 31) / 32 * tile;
   if (p->split > 1) p->p_bytes = (size_t)p->split * M * N * 4;
   return p->x_bytes + p->p_bytes <= kGemmScratchBytes;
 }

@@ -217,3 +217,29 @@ def test_captured_8_bit_prefills(n, k, m, kernel):
     4096, 2048 tokens 441 us against 577); K % 64 != 0 has one only."""
     for row in fake_hip.call(__name__, "plans", 8, n, k, [m], ["capture"]):
         assert _names(row["capture"]) == [kernel]
+
+
+def grids(hip, pe, bits, n, k, m, how):
+    ctx = pe.Context(0)
+    w = ctx.upload_dev(fake_hip.Tensor(hip, payload_bytes(n, k, bits)), n, k, bits)
+    x, y = fake_hip.Tensor(hip, m * k * 2), fake_hip.Tensor(hip, m * n * 2)
+    hip.clear()
+    hip.lib.fake_set_capturing(STREAM if how == "capture" else None)
+    ctx.gemm_dev(w, x, m, y, None if how == "own" else STREAM)
+    return [[ln.name, ln.grid[0] * ln.threads, ln.lk.M if ln.lk else 0, (ln.lk.Y - y.address) // (2 * n) if ln.lk else 0]
+            for ln in hip.launches]
+
+
+@pytest.mark.parametrize("how", ["own", "lent", "capture"])
+@pytest.mark.parametrize("bits,n,k,m", [(8, 151936, 904, 150_001), (4, 151936, 904, 150_001), (8, 1_000_003, 8, 40_000)])
+def test_launches_of_less_than_2_32_threads(bits, n, k, m, how):
+    """More outputs than one launch has threads for: several, of some tokens each,
+    that cover every token once."""
+    got = fake_hip.call(__name__, "grids", bits, n, k, m, how)
+    assert all(x[1] < 1 << 32 for x in got), got
+    at = 0
+    for name, _, tokens, first in got:
+        if "k_gemm_lookup" in name:
+            assert first == at
+            at += tokens
+    assert at == m
